@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <float.h>
+#include <limits.h>
 #include <stdint.h>
 #include <string.h>
 
@@ -156,6 +157,12 @@ template <int KIND, bool FWD> __device__ __forceinline__ void xf8(float *v) {
         v[4] = (q + u3) + (r + a6); v[5] = (q + u3) + (r - a6);
         v[6] = (q - u3) - (s - a7); v[7] = (q - u3) - (s + a7);
     }
+}
+
+// Orders the LDS accesses of one wave: they execute in order, so only the compiler is held back.
+__device__ __forceinline__ void lds_order() {
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
 }
 
 __device__ __forceinline__ float tree8(const float *c) {
@@ -549,6 +556,52 @@ __device__ __forceinline__ void lds_step(float (&w)[9][8], const char *lds, cons
     insert8<false>(L, row_ok && (unsigned)xt <= (unsigned)(W - 8) ? e : FLT_MAX, (unsigned)xt | ybits, 0);
 }
 
+// Scans columns x0 .. x0 + span of rows y + dy .. y + dy_end - 1 in a staged region whose row 0 is ry0; X0 is x0 there.
+template <int M>
+__device__ __forceinline__ void lds_scan(const float *region, int LS, int X0, int ry0, int W, int H, int x0, int y,
+                                         int span, int dy, int dy_end, const RefPatch &R, List8 &L) {
+    const char *lds = reinterpret_cast<const char *>(region);
+    for (; dy < dy_end; ++dy) {
+        const int yy = y + dy;
+        const bool row_ok = yy >= 0 && yy <= H - 8;
+        const unsigned ybits = (unsigned)yy << 16;
+        int vo[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) vo[r] = (lds_row(yy + r - ry0, LS) + X0) * 4;
+        float w[9][8];
+        lds_col<0>(w[0], lds, vo);
+        lds_col<4>(w[1], lds, vo);
+        lds_col<8>(w[2], lds, vo);
+        lds_col<12>(w[3], lds, vo);
+        lds_col<16>(w[4], lds, vo);
+        lds_col<20>(w[5], lds, vo);
+        lds_col<24>(w[6], lds, vo);
+        lds_col<28>(w[7], lds, vo);
+        for (int tb = 0; tb <= span; tb += 9) {
+            const int xt = x0 + tb;
+            lds_step<M, 0>(w, lds, vo, W, xt + 0, row_ok, ybits, R, L);
+            if (tb + 1 > span) break;
+            lds_step<M, 1>(w, lds, vo, W, xt + 1, row_ok, ybits, R, L);
+            if (tb + 2 > span) break;
+            lds_step<M, 2>(w, lds, vo, W, xt + 2, row_ok, ybits, R, L);
+            if (tb + 3 > span) break;
+            lds_step<M, 3>(w, lds, vo, W, xt + 3, row_ok, ybits, R, L);
+            if (tb + 4 > span) break;
+            lds_step<M, 4>(w, lds, vo, W, xt + 4, row_ok, ybits, R, L);
+            if (tb + 5 > span) break;
+            lds_step<M, 5>(w, lds, vo, W, xt + 5, row_ok, ybits, R, L);
+            if (tb + 6 > span) break;
+            lds_step<M, 6>(w, lds, vo, W, xt + 6, row_ok, ybits, R, L);
+            if (tb + 7 > span) break;
+            lds_step<M, 7>(w, lds, vo, W, xt + 7, row_ok, ybits, R, L);
+            if (tb + 8 > span) break;
+            lds_step<M, 8>(w, lds, vo, W, xt + 8, row_ok, ybits, R, L);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) vo[r] += 36;
+        }
+    }
+}
+
 // WR wave rows: a workgroup of 128 * WR lanes. SPLIT lanes share a block: each scans a
 // contiguous band of its search rows, and the later bands' sorted lists are inserted into the
 // earlier ones with the same strict-< rule, which reproduces one sequential scan exactly. A wave
@@ -588,51 +641,9 @@ __device__ __forceinline__ void match_lds_body(const MatchArgs &a, int tile, flo
     List8 L;
     list_init<false>(L, 0);
 
-    const char *lds = reinterpret_cast<const char *>(region);
-    const int span = 2 * Rg;
-    const int X0 = x - Rg - rx0;
     const int nrows = 2 * Rg + 1;
-    const int dy_end = -Rg + (nrows * (part + 1)) / SPLIT;
-    for (int dy = -Rg + (nrows * part) / SPLIT; dy < dy_end; ++dy) {
-        const int yy = y + dy;
-        const bool row_ok = yy >= 0 && yy <= H - 8;
-        const unsigned ybits = (unsigned)yy << 16;
-        int vo[8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) vo[r] = (lds_row(yy + r - ry0, LS) + X0) * 4;
-        float w[9][8];
-        lds_col<0>(w[0], lds, vo);
-        lds_col<4>(w[1], lds, vo);
-        lds_col<8>(w[2], lds, vo);
-        lds_col<12>(w[3], lds, vo);
-        lds_col<16>(w[4], lds, vo);
-        lds_col<20>(w[5], lds, vo);
-        lds_col<24>(w[6], lds, vo);
-        lds_col<28>(w[7], lds, vo);
-        const int x0 = x - Rg;
-        for (int tb = 0; tb <= span; tb += 9) {
-            const int xt = x0 + tb;
-            lds_step<M, 0>(w, lds, vo, W, xt + 0, row_ok, ybits, R, L);
-            if (tb + 1 > span) break;
-            lds_step<M, 1>(w, lds, vo, W, xt + 1, row_ok, ybits, R, L);
-            if (tb + 2 > span) break;
-            lds_step<M, 2>(w, lds, vo, W, xt + 2, row_ok, ybits, R, L);
-            if (tb + 3 > span) break;
-            lds_step<M, 3>(w, lds, vo, W, xt + 3, row_ok, ybits, R, L);
-            if (tb + 4 > span) break;
-            lds_step<M, 4>(w, lds, vo, W, xt + 4, row_ok, ybits, R, L);
-            if (tb + 5 > span) break;
-            lds_step<M, 5>(w, lds, vo, W, xt + 5, row_ok, ybits, R, L);
-            if (tb + 6 > span) break;
-            lds_step<M, 6>(w, lds, vo, W, xt + 6, row_ok, ybits, R, L);
-            if (tb + 7 > span) break;
-            lds_step<M, 7>(w, lds, vo, W, xt + 7, row_ok, ybits, R, L);
-            if (tb + 8 > span) break;
-            lds_step<M, 8>(w, lds, vo, W, xt + 8, row_ok, ybits, R, L);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) vo[r] += 36;
-        }
-    }
+    lds_scan<M>(region, LS, x - Rg - rx0, ry0, W, H, x - Rg, y, 2 * Rg, -Rg + (nrows * part) / SPLIT,
+                -Rg + (nrows * (part + 1)) / SPLIT, R, L);
 
     // merge the bands in scan order: (0 <- 1, 2 <- 3), then 0 <- 2
 #pragma unroll
@@ -845,6 +856,947 @@ __global__ __launch_bounds__(256) void k_match_lds4(MatchArgs a) {
     zero_share(a);
 }
 
+// ---- screened search (ssd) ---------------------------------------------------------------------
+// The distance of a block to a candidate is |a|^2 + |b|^2 - 2 a.b, and a.b over all candidates of a
+// block is a matrix product. The screen computes it on the matrix cores from half-precision copies
+// of the pixels, derives per block a threshold that every one of its 8 best candidates is proven to
+// pass (about 9 of 1089 do on video with noise), and only those are evaluated exactly, in FP32 and in
+// the reference's order of operations. Lists and distances are those of the exhaustive scan.
+//
+// A workgroup is one wave and owns 4 x 4 blocks (the 16 rows of a product). Products run on
+// v_mfma_f32_16x16x32_f16: lane l, i = l%16, g = l/16, holds A[i][8g..8g+7], B[8g..8g+7][i] and
+// D[4g..4g+3][i]. Row 4*gy + qx of A is the block at (qx, gy) of the 4 x 4, so a lane's four results
+// are four blocks of one block row at one candidate. k = 8g + c is pixel column c of the g-th image row of a
+// group of four: B of a 4-row group is loaded once and serves every candidate row that
+// touches it, by products with copies of A shifted by s = 0..3 rows and zero elsewhere (11 shifted
+// fragments, one set of 4 candidate rows).
+//
+// Bounds. Pixels are centred on the mean of the wave's own blocks (flat areas, where distances are
+// smallest, then have the smallest halves and the finest steps), scaled by a power of two and
+// rounded to half (subnormal halves may count as 0), with d = half a step of the largest half that the
+// block or a candidate this near can hold (screen_eps). With S the distance of two patches and S_q that of their rounded copies,
+// |sqrt(S) - sqrt(S_q)| <= 2 sqrt(64) d = eps. A computed S' = n_a - 2 (a.b - n_b/2) differs from S_q
+// by the accumulation's rounding. One product instruction was measured to be off by at most 9.3 units
+// of 2^-24 of its largest term or result (one term 2^12 times the other 31, all truncated; 2 to 4 for terms of
+// like size); 17 is what truncating every term at half a unit gives, and 3 instructions make
+// |S' - S_q| <= c (n_a + n_b) with c = 8e-6, the norms' own rounding included, and n_b <= 2 n_a + 2 S_q.
+// Pass 1 finds a T' that 8 distinct candidates do not exceed; their exact distances, hence the 8
+// best, are below (sqrt((T' + 3c n_a)(1 + 3c)) + eps)^2, up to FP32 rounding; a candidate below that has
+// S' <= T'' (screen_limit). Pass 2 recomputes the products and passes on candidates with S' <= T''.
+// Queues are bounded: a full one is evaluated at once and the exact 8th distance tightens T''. A tile with
+// more than kScrMost candidates to evaluate, or with non-finite values, is marked and left to k_match_tied, which
+// searches it exhaustively: at about 130 cycles per gathered candidate, a wave that evaluated all of a tied
+// window took up to 570 k cycles (a usual one takes 50 to 97 k) and a small frame waited for it alone.
+//
+// What bounds it: VALU issue, about 30 instructions per candidate row of 16 blocks in pass 1 and 40 in
+// pass 2 with the products (11 per 4 rows and 16 columns, 16 cycles each) beside them, then the latency of
+// the exact evaluations (144 candidates per 16 blocks, gathered from L2). Two waves per SIMD: 256 VGPRs hold the 11
+// fragments of A, three groups of B and three sets of accumulators, and a wave's LDS stays within an
+// eighth of the CU's. 4 x 4 blocks waste least of a product (window + 3 block steps per axis), and one wave
+// per workgroup needs no barrier and centres its pixels by itself. 1920x1080 at block_step 4, bm_range 16:
+// 358 us by the shared-column scan, 155 here; block_step 2, bm_range 16: 1758 and 506; 640x360 at block_step 4, bm_range 16: 155 and 32
+// (k_match_tied, with no tile to search, adds 3).
+typedef unsigned vsz_u2 __attribute__((ext_vector_type(2)));
+typedef unsigned vsz_u4 __attribute__((ext_vector_type(4)));
+typedef _Float16 scr_h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 scr_h2 __attribute__((ext_vector_type(2)));
+typedef float scr_f2 __attribute__((ext_vector_type(2)));
+typedef float scr_f4 __attribute__((ext_vector_type(4)));
+
+constexpr int kScrMost = 384;  // candidates evaluated per wave (144 and up; on video with noise below 200)
+constexpr int kScrCap = 16;    // keys kept per block between two insertions
+constexpr int kScrLds8 = 20480;   // LDS bytes that each of 8 workgroups of a CU may take
+constexpr int kScrLdsMax = 40960;  // a quarter of the CU's
+
+struct ScreenGeom {
+    int ng, tiles;        // 4-row groups and 16-column tiles of a 4 x 4 block tile's candidates
+    int pw, ph, nc, nr;   // half-pixel region (pitch, rows); norm array (pitch, rows)
+    int queue;            // 8-byte results a wave can queue
+    int slack;            // zeroed halves past the region: reads of masked columns in its last row end there
+    int half_bytes, norm_bytes;
+    // how 64 lanes walk the region's pairs and the norms' segments: i / d = i * m >> 16 below 4096
+    int rstep, pair_m, segs, segs_m, vsegs, vsegs_m;
+};
+
+struct ScreenWave {  // per wave
+    unsigned long long kbuf[16 * kScrCap];  // (distance, position) keys to insert, per block
+    unsigned long long best[16 * 8];        // sorted keys of the best so far
+    unsigned cnt[16];
+    unsigned refpos[16];
+};
+
+// Bytes of the half region and of the norms (the last 8 rows of their first stage reach into the rest,
+// which is not in use yet).
+inline int screen_half_bytes(const ScreenGeom &G) { return ((G.pw * G.ph + G.slack) * 2 + 15) & ~15; }
+inline int screen_norm_bytes(const ScreenGeom &G) { return (G.nc * G.nr * 4 + 15) & ~15; }
+inline int screen_lds_bytes(const ScreenGeom &G) {
+    const int tail = 8 * G.nc * 4, rest = (int)sizeof(ScreenWave) + 8 * G.queue + 8;
+    return screen_half_bytes(G) + screen_norm_bytes(G) + (tail > rest ? tail : rest);
+}
+
+inline ScreenGeom screen_geom(int bs, int R, int nt) {
+    ScreenGeom G;
+    const int span = 3 * bs + 2 * R + 1;
+    G.ng = (span + 3) / 4;
+    G.tiles = ((span + 15) / 16 + nt - 1) / nt * nt;
+    G.pw = (span + 7 + 3) & ~3;   // columns past it belong to masked candidates only (they read on)
+    G.nc = (span + 1) & ~1;
+    if (G.nc % 16 == 0) G.nc += 2;   // rows of one column 12 apart in different banks
+    G.nr = 4 * G.ng;
+    G.ph = G.nr + 8;
+    G.slack = (16 * G.tiles + 64 - G.pw + 7) / 8 * 8;
+    G.slack = G.slack > 64 ? G.slack : 64;
+    G.half_bytes = screen_half_bytes(G);
+    G.norm_bytes = screen_norm_bytes(G);
+    const auto magic = [](int d) { return (65536 + d - 1) / d; };
+    G.rstep = G.pw / 2 <= 64 ? 64 / (G.pw / 2) : 1;
+    G.pair_m = magic(G.pw / 2 <= 64 ? G.pw / 2 : 64);
+    G.segs = (G.nc + 23) / 24;
+    G.segs_m = magic(G.segs);
+    G.vsegs = (G.nr + 11) / 12;
+    G.vsegs_m = magic(G.vsegs);
+    // the queue takes what is left of the LDS that lets 8 workgroups share a CU
+    G.queue = 256;
+    const int room = kScrLds8 - screen_lds_bytes(G);
+    G.queue += (room < 0 ? 0 : room > 8 * 64 ? 8 * 64 : room) / 8;
+    return G;
+}
+
+template <int CTRL> __device__ __forceinline__ int dpp_i(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL> __device__ __forceinline__ float dpp_f(float v) { return __int_as_float(dpp_i<CTRL>(__float_as_int(v))); }
+template <int CTRL> __device__ __forceinline__ double dpp_d(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)dpp_i<CTRL>((int)(unsigned)u), hi = (unsigned)dpp_i<CTRL>((int)(unsigned)(u >> 32));
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+constexpr int kDppRor4 = 0x124, kDppRor8 = 0x128;
+
+// Keys (distance bits << 32 | y << 16 | x) of non-negative finite distances order as doubles (the
+// reference's strict-< rule: equal distances by scan order); one instruction each, bits preserved.
+__device__ __forceinline__ double key_min(double a, double b) {
+    double d;
+    asm("v_min_f64 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+    return d;
+}
+__device__ __forceinline__ double key_max(double a, double b) {
+    double d;
+    asm("v_max_f64 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+    return d;
+}
+__device__ __forceinline__ void key_insert(double (&L)[8], double k) {
+#pragma unroll
+    for (int i = 7; i > 0; --i) L[i] = key_max(L[i - 1], key_min(L[i], k));
+    L[0] = key_min(L[0], k);
+}
+// The 8 smallest of two sorted lists, sorted.
+template <int CTRL> __device__ __forceinline__ void key_merge(double (&L)[8]) {
+    double b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) b[i] = dpp_d<CTRL>(L[i]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) L[i] = key_min(L[i], b[7 - i]);
+#pragma unroll
+    for (int d = 4; d > 0; d >>= 1)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (!(i & d)) {
+                const double lo = key_min(L[i], L[i + d]), hi = key_max(L[i], L[i + d]);
+                L[i] = lo;
+                L[i + d] = hi;
+            }
+}
+
+// Floats as integers of the same order (its own inverse).
+__device__ __forceinline__ int ordered(int v) { return v ^ ((v >> 31) & 0x7fffffff); }
+
+__device__ __forceinline__ void bitonic8_desc(int (&v)[8]) {
+#pragma unroll
+    for (int d = 4; d > 0; d >>= 1)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (!(i & d)) {
+                const int hi = max(v[i], v[i + d]), lo = min(v[i], v[i + d]);
+                v[i] = hi;
+                v[i + d] = lo;
+            }
+}
+
+// For each q, the 8th largest of the 64 values m[0..3][q] of a row of 16 lanes.
+__device__ __forceinline__ void eighth_of_64(const float (&m)[4][4], int lane, float (&out)[4]) {
+    int L[8];   // lane l of a quad goes on with the quad's list of q = l & 3
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int a = ordered(__float_as_int(m[0][q])), b = ordered(__float_as_int(m[1][q]));
+        const int c = ordered(__float_as_int(m[2][q])), d = ordered(__float_as_int(m[3][q]));
+        const int ab = max(a, b), ba = min(a, b), cd = max(c, d), dc = min(c, d);
+        const int mid = min(ab, cd), w = max(ba, dc);
+        int v[8] = {max(ab, cd), max(mid, w), min(mid, w), min(ba, dc)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[4 + i] = dpp_i<kDppXor1>(v[3 - i]);
+        bitonic8_desc(v);
+        int o[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = max(v[i], dpp_i<kDppXor2>(v[7 - i]));
+        bitonic8_desc(o);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) L[i] = q == 0 || (lane & 3) == q ? o[i] : L[i];
+    }
+    int o[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = max(L[i], dpp_i<kDppRor4>(L[7 - i]));
+    bitonic8_desc(o);
+    int r = max(o[0], dpp_i<kDppRor8>(o[7]));
+#pragma unroll
+    for (int i = 1; i < 8; ++i) r = min(r, max(o[i], dpp_i<kDppRor8>(o[7 - i])));
+    r = ordered(r);
+    out[0] = __int_as_float(dpp_i<0x00>(r));
+    out[1] = __int_as_float(dpp_i<0x55>(r));
+    out[2] = __int_as_float(dpp_i<0xAA>(r));
+    out[3] = __int_as_float(dpp_i<0xFF>(r));
+}
+
+constexpr float kScrC = 8e-6f;
+
+// eps for patches whose pixels stay below m: half a step of such a half, what a subnormal half may lose,
+// the centring's rounding; `floor` is what FP32 distances lose below the normal range.
+__device__ __forceinline__ float screen_eps(float m, float floor) {
+    return 16.0f * (__builtin_ldexpf(1.0f, __builtin_amdgcn_frexp_expf(m) - 12) + 6.2e-5f + 1.2e-7f * m) + floor;
+}
+// The largest S' of a candidate whose S_q is at most u (n: the block's squared norm).
+__device__ __forceinline__ float screen_limit(float u, float n) {
+    return u * (1.0f + 6.0f * kScrC) + 3.1f * kScrC * n + 1.0e-5f;
+}
+
+// 8 consecutive halves from index h of a dword-aligned LDS array; sh = 16 * (h & 1).
+__device__ __forceinline__ scr_h8 lds_halves(const unsigned *base, int h, unsigned sh) {
+    const unsigned *p = base + (h >> 1);
+    unsigned w[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) w[i] = p[i];
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    u4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], sh);
+    return __builtin_bit_cast(scr_h8, o);
+}
+
+__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
+// Largest value of a wave; NaN if any is.
+__device__ __forceinline__ float wave_max(float v) {
+    v = max_nan(v, dpp_f<kDppXor1>(v));
+    v = max_nan(v, dpp_f<kDppXor2>(v));
+    v = max_nan(v, dpp_f<kDppHalfMirror>(v));
+    v = max_nan(v, dpp_f<kDppMirror>(v));
+    const int i = __float_as_int(v);
+    return max_nan(max_nan(__int_as_float(__builtin_amdgcn_readlane(i, 0)), __int_as_float(__builtin_amdgcn_readlane(i, 16))),
+                   max_nan(__int_as_float(__builtin_amdgcn_readlane(i, 32)), __int_as_float(__builtin_amdgcn_readlane(i, 48))));
+}
+
+__device__ __forceinline__ int wave_sum(int v) {
+    v += dpp_i<kDppXor1>(v);
+    v += dpp_i<kDppXor2>(v);
+    v += dpp_i<kDppHalfMirror>(v);
+    v += dpp_i<kDppMirror>(v);
+    return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
+           __builtin_amdgcn_readlane(v, 48);
+}
+
+template <int NT>
+__device__ __forceinline__ void match_screen_body(const MatchArgs &a, const ScreenGeom &G, int tile, float *smem) {
+    const int lane = threadIdx.x & 63;
+    const int W = a.width, H = a.height, S = a.stride, bs = a.block_step, R = a.bm_range;
+    unsigned *hw = reinterpret_cast<unsigned *>(smem);                       // half pairs
+    float *nh = smem + (G.half_bytes >> 2);                                 // n_b, infinite outside the plane
+    ScreenWave *ws = reinterpret_cast<ScreenWave *>(reinterpret_cast<char *>(nh) + G.norm_bytes);
+    // queue: a lane's passing results of a 4-row group (its low 24 bits of each word, two rows a word), with
+    // the lane and the group above them; while it is emptied, its first part takes the list of candidates
+    vsz_u2 *queue = reinterpret_cast<vsz_u2 *>(ws + 1);
+    unsigned *list = reinterpret_cast<unsigned *>(queue);
+    const PlaneBuf img = make_plane_buf(a.img, (unsigned)(a.ts * 4));
+
+    const int n = lane & 15, g = lane >> 4;
+    const int bxm = tile % a.tiles_x * 4, bym = tile / a.tiles_x * 4;      // the wave's 4 x 4 blocks
+    const int xm = min(bxm * bs, W - 8), ym = min(bym * bs, H - 8);
+    const int rx0 = xm - R, ry0 = ym - R;                                    // the region's corner
+    const int xr_n = min(min(bxm + (n & 3), a.nbx - 1) * bs, W - 8);         // block n & 3, n >> 2
+    const int yr_n = min(min(bym + (n >> 2), a.nby - 1) * bs, H - 8);
+
+    // -- the region in half precision (pixels outside the plane stand for the nearest inside: only
+    //    invalid candidates read them) ----------------------------------------------------------------
+    const int p2 = G.pw >> 1, rstep = G.rstep;
+    const int srow = lane * G.pair_m >> 16, spair = lane - srow * p2;   // row 0 if a row has 64 pairs or more
+    float mid = buf_load_s(img, ((yr_n + 3) * S + xr_n + 3) * 4, 0);
+    const bool inside = rx0 >= 0 && rx0 + G.pw <= W && ry0 >= 0 && ry0 + G.ph <= H;
+    // d = (v - mid) * sc in one rounding (sc is a power of two); the largest |d|
+    const auto convert = [&](float sc, bool bad) -> float {
+        constexpr int kRows = 28;
+        const float off = -mid * sc;
+        float big = 0.0f;
+        for (int pr = spair; pr < p2; pr += 64) {
+            const int gx = rx0 + 2 * pr;
+            for (int r = srow; r < (srow < rstep ? G.ph : 0); r += kRows * rstep) {
+                float v[kRows][2];
+                if (inside) {   // rows past the region's end are inside the plane's buffer or read as 0
+                    const int at = ((ry0 + r) * S + gx) * 4, step = rstep * S * 4;
+#pragma unroll
+                    for (int k = 0; k < kRows; ++k) {
+                        const vsz_u2 u = __builtin_bit_cast(vsz_u2, __builtin_amdgcn_raw_buffer_load_b64(img.rsrc, at, k * step, 0));
+                        v[k][0] = __uint_as_float(u[0]);
+                        v[k][1] = __uint_as_float(u[1]);
+                    }
+                } else {
+                    const int x0 = 4 * min(max(gx, 0), W - 1), x1 = 4 * min(max(gx + 1, 0), W - 1);
+#pragma unroll
+                    for (int k = 0; k < kRows; ++k) {
+                        const int gy = min(max(ry0 + r + k * rstep, 0), H - 1) * S * 4;
+                        v[k][0] = buf_load_s(img, gy + x0, 0);
+                        v[k][1] = buf_load_s(img, gy + x1, 0);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < kRows; ++k)
+                    if (r + k * rstep < G.ph) {
+                        const float d0 = fmaf(v[k][0], sc, off), d1 = fmaf(v[k][1], sc, off);
+                        big = max_nan(max_nan(big, fabsf(d0)), fabsf(d1));
+                        const scr_h2 q = {(_Float16)d0, (_Float16)d1};
+                        hw[(r + k * rstep) * p2 + pr] = bad ? 0u : __builtin_bit_cast(unsigned, q);
+                    }
+            }
+        }
+        return wave_max(big);
+    };
+    for (int i = lane; i < G.slack >> 1; i += 64) hw[(G.pw * G.ph >> 1) + i] = 0u;
+    mid += dpp_f<kDppXor1>(mid);
+    mid += dpp_f<kDppXor2>(mid);
+    mid += dpp_f<kDppHalfMirror>(mid);
+    mid += dpp_f<kDppMirror>(mid);
+    mid = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mid * 0.0625f)));
+    float sc = 1024.0f, big;
+    bool bad = false;
+    for (bool again = false;; again = true) {
+        big = convert(sc, bad);
+        if (again || (big < 60000.0f && !(big < 8.0f && big > 0.0f))) break;
+        // not the range of video: scale the largest to 512..1024; without a finite one, no screening
+        const float top = big * (1.0f / 1024.0f);
+        bad = !(top < 1.0e37f);
+        sc = bad ? 1.0f : __builtin_ldexpf(1.0f, min(10 - __builtin_amdgcn_frexp_expf(top), 120));
+    }
+    const bool flat = big == 0.0f && !bad;
+    if (lane < 16) {
+        ws->refpos[lane] = pack_xy(xr_n, yr_n);
+        ws->cnt[lane] = 0u;
+    }
+    lds_order();
+
+    bool tied = bad;   // left to k_match_tied
+    if (!flat && !tied) {
+        const float eps_floor = 1.0e-21f * sc;
+
+        // -- norms: horizontal 8-sums of squares, then vertical ones in place ----------------------
+        const int segs = G.segs;
+        for (int i0 = lane; i0 < segs * G.ph; i0 += 128) {
+            vsz_u2 u[2][8];
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {   // past the end: the last segment again
+                const int i = min(i0 + 64 * v, segs * G.ph - 1), r = i * G.segs_m >> 16, c0 = (i - r * segs) * 24;
+                const vsz_u2 *p = reinterpret_cast<const vsz_u2 *>(hw + ((r * G.pw + c0) >> 1));   // pw % 4 == 0
+#pragma unroll
+                for (int k = 0; k < 8; ++k) u[v][k] = p[k];
+            }
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                const int i = min(i0 + 64 * v, segs * G.ph - 1), r = i * G.segs_m >> 16, c0 = (i - r * segs) * 24;
+                float s[30];
+#pragma unroll
+                for (int k = 0; k < 15; ++k) {
+                    const unsigned a0 = u[v][k >> 1][k & 1], a1 = u[v][(k + 1) >> 1][(k + 1) & 1];
+                    const scr_h2 q = __builtin_bit_cast(scr_h2, a0);
+                    const scr_h2 o = __builtin_bit_cast(scr_h2, __builtin_amdgcn_alignbit(a1, a0, 16));
+                    s[2 * k] = __builtin_amdgcn_fdot2(q, q, 0.0f, false);
+                    s[2 * k + 1] = __builtin_amdgcn_fdot2(o, o, 0.0f, false);
+                }
+#pragma unroll
+                for (int k = 0; k < 28; ++k) s[k] += s[k + 2];
+#pragma unroll
+                for (int k = 0; k < 24; ++k) s[k] += s[k + 4];
+                scr_f2 *o = reinterpret_cast<scr_f2 *>(nh + r * G.nc + c0);   // rows and segments start at 8 bytes
+#pragma unroll
+                for (int k = 0; k < 12; ++k)
+                    if (c0 + 2 * k < G.nc) o[k] = scr_f2{s[2 * k], s[2 * k + 1]};
+            }
+        }
+        lds_order();
+        const int vsegs = G.vsegs, vcols = 64 * G.vsegs_m >> 16;
+        const int vc = lane * G.vsegs_m >> 16, r0 = (lane - vc * vsegs) * 12;
+        for (int c1 = vc; c1 < G.nc; c1 += 3 * vcols) {
+            float s[3][19];
+#pragma unroll
+            for (int v = 0; v < 3; ++v) {
+                const float *col = nh + r0 * G.nc + min(c1 + v * vcols, G.nc - 1);
+#pragma unroll
+                for (int k = 0; k < 19; ++k) s[v][k] = col[k * G.nc];   // past the last row: never used
+            }
+            lds_order();
+#pragma unroll
+            for (int v = 0; v < 3; ++v) {
+#pragma unroll
+                for (int k = 0; k < 18; ++k) s[v][k] += s[v][k + 1];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) s[v][k] += s[v][k + 2];
+#pragma unroll
+                for (int k = 0; k < 12; ++k) s[v][k] += s[v][k + 4];
+                // rows past the array go where its first stage's last rows were
+                const int c = c1 + v * vcols, y0 = ry0 + r0;
+                float *o = nh + r0 * G.nc + c;
+                if (vc < vcols && c < G.nc) {
+                    if (inside) {
+#pragma unroll
+                        for (int k = 0; k < 12; ++k) o[k * G.nc] = s[v][k];
+                    } else {
+                        const bool cin = rx0 + c >= 0 && rx0 + c <= W - 8;
+#pragma unroll
+                        for (int k = 0; k < 12; ++k)
+                            o[k * G.nc] = cin && (unsigned)(y0 + k) <= (unsigned)(H - 8) ? s[v][k] : __builtin_inff();
+                    }
+                }
+            }
+            lds_order();
+        }
+
+        int dxq[4];                                          // blocks' offsets from the tile's first
+#pragma unroll
+        for (int q = 0; q < 4; ++q) dxq[q] = min(min(bxm + q, a.nbx - 1) * bs, W - 8) - xm;
+        const int dyg = min(min(bym + g, a.nby - 1) * bs, H - 8) - ym;   // block row of this lane's results
+        const unsigned dy_span = bym + g < a.nby ? 2u * (unsigned)R : 0u;   // (a row past the last block's: none but one candidate row)
+        const unsigned long long kFill = (unsigned long long)__float_as_uint(FLT_MAX) << 32;
+        ws->best[lane] = kFill;
+        ws->best[64 + lane] = kFill;
+
+        // A: row n is the block (n & 3, n >> 2)
+        scr_h8 A[4][3];
+        const auto loadA = [&]() {
+            const int xr = xr_n - rx0, yr = yr_n - ry0;
+            const scr_h8 z = {};
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int part = 0; part < 3; ++part) {
+                    if (s == 0 && part == 2) continue;
+                    const int row = 4 * part + g - s;
+                    const bool on = row >= 0 && row < 8;
+                    const scr_h8 v = lds_halves(hw, (yr + (on ? row : 0)) * G.pw + xr, (xr & 1) * 16);
+                    A[s][part] = on ? v : z;
+                }
+        };
+        loadA();
+        // squared norms of this lane's four result rows' blocks
+        float na[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) na[q] = nh[(dyg + R) * G.nc + dxq[q] + R];
+
+        const int chunks = G.tiles / NT;
+        const int j0 = max(0, -ry0) >> 2;                                  // groups that meet the plane
+        const int j1 = min(G.ng, (H - 8 - ry0) / 4 + 1);
+        const float inf = __builtin_inff();
+        const unsigned bsh = (n & 1) * 16;
+
+        float m[4][4];   // largest a.b - n_b/2 of this lane's candidates, by row mod 4 and block
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) m[s][q] = -inf;
+        float sub[NT][4];   // pass 1: 0, pass 2: the least a.b - n_b/2 that passes; infinite outside the window
+
+        const auto mask_cols = [&](int xs, const float (&th)[4]) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int dx = xs + 16 * t + n - dxq[q];
+                    sub[t][q] = dx >= 0 && dx <= 2 * R && bxm + q < a.nbx ? th[q] : inf;
+                }
+        };
+        struct Raw {   // a 4-row group as read, and the norms of one
+            unsigned b[NT][5];
+        };
+        const auto read_b = [&](int j, int xs, Raw &v) {
+            const unsigned *p = hw + (((4 * j + g) * G.pw + xs + n) >> 1);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 5; ++i) v.b[t][i] = p[8 * t + i];
+        };
+        const auto align_b = [&](const Raw &v, scr_h8 (&B)[NT]) {
+            typedef unsigned u4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                u4 o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_alignbit(v.b[t][i + 1], v.b[t][i], bsh);
+                B[t] = __builtin_bit_cast(scr_h8, o);
+            }
+        };
+        const auto read_nh = [&](int row, int xs, float (&h)[NT]) {
+            const float *hp = nh + row * G.nc + xs + n;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) h[t] = hp[16 * t];
+        };
+        // Walks groups j.. of the chunk at xs. A row's results are a.b - n_b/2 - sub: prep() loads -n_b/2 - sub
+        // into the accumulators, multiply() adds the products. While a row's products run, the next row
+        // is prepared and the row before is used; three sets of accumulators take turns (12 rows are three
+        // groups). The LDS reads of a group are issued a group ahead. use(j, s, acc) takes a row's results,
+        // more() says whether to go on.
+        const auto walk = [&](int &j, int xs, const auto &use, const auto &more) {
+            scr_h8 B0[NT], B1[NT], B2[NT];
+            float h[4][NT];
+            scr_f4 acc[3][NT];
+            const auto prep = [&](int row, const float (&hr)[NT], scr_f4 (&o)[NT]) {   // rows from ym - R
+                const bool yok = (unsigned)(row - dyg) <= dy_span;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const float hv = yok ? hr[t] : inf;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) o[t][q] = fmaf(hv, -0.5f, -sub[t][q]);
+                }
+            };
+            {
+                Raw v;
+                read_b(j, xs, v);
+                align_b(v, B0);
+                read_b(j + 1, xs, v);
+                align_b(v, B1);
+                read_b(j + 2, xs, v);
+                align_b(v, B2);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) read_nh(4 * j + s, xs, h[s]);
+            }
+            prep(4 * j, h[0], acc[0]);
+            read_nh(4 * j + 4, xs, h[0]);
+            const auto step = [&](auto first, scr_h8 (&C0)[NT], scr_h8 (&C1)[NT], scr_h8 (&C2)[NT]) {
+                constexpr int F = decltype(first)::value;   // the set of row 0
+                Raw v;
+                read_b(j + 3, xs, v);
+                const auto row = [&](auto sc_) {
+                    constexpr int s = decltype(sc_)::value;
+                    scr_f4 (&c)[NT] = acc[(F + s) % 3];
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) c[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s][0], C0[t], c[t], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) c[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s][1], C1[t], c[t], 0, 0, 0);
+                    if constexpr (s > 0)
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) c[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s][2], C2[t], c[t], 0, 0, 0);
+                    prep(4 * j + s + 1, h[(s + 1) & 3], acc[(F + s + 1) % 3]);
+                    read_nh(4 * j + s + 5, xs, h[(s + 1) & 3]);
+                    if constexpr (s > 0) use(j, std::integral_constant<int, s - 1>{}, acc[(F + s + 2) % 3]);
+                };
+                row(std::integral_constant<int, 0>{});
+                row(std::integral_constant<int, 1>{});
+                row(std::integral_constant<int, 2>{});
+                row(std::integral_constant<int, 3>{});
+                align_b(v, C0);
+                use(j, std::integral_constant<int, 3>{}, acc[F % 3]);
+                // one product, then three of the other vector instructions
+#pragma unroll
+                for (int i = 0; i < 11 * NT; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                ++j;
+                return more();
+            };
+            for (;;) {
+                if (!step(std::integral_constant<int, 0>{}, B0, B1, B2)) break;
+                if (!step(std::integral_constant<int, 1>{}, B1, B2, B0)) break;
+                if (!step(std::integral_constant<int, 2>{}, B2, B0, B1)) break;
+            }
+        };
+
+        // -- pass 1 ----------------------------------------------------------------------------------
+        {
+            const float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int ch = 0; ch < chunks; ++ch) {
+                const int xs = 16 * NT * ch;          // first column of the chunk, from xm - R
+                mask_cols(xs, zero);
+                int j = j0;
+                walk(j, xs, [&](int, auto sc_, const scr_f4 (&acc)[NT]) {
+                    constexpr int s = decltype(sc_)::value;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        float v = m[s][q];
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) v = max_nan(v, acc[t][q]);
+                        m[s][q] = v;
+                    }
+                }, [&] { return j < j1; });
+            }
+        }
+        // The largest S' of a candidate whose exact distance has a root of at most re: its pixels differ
+        // from the block's by no more than that, so they stay below |block| + re.
+        float rna[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) rna[q] = __builtin_amdgcn_sqrtf(na[q]) * 1.000001f;
+        const auto near_limit = [&](float re, int q) {
+            const float rt = re + screen_eps(fminf(big, (rna[q] + re) * 1.001f), eps_floor);
+            return screen_limit(rt * rt * 1.00001f, na[q]);
+        };
+        float th[4];
+        {
+            float tau[4];
+            eighth_of_64(m, lane, tau);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float t1 = fmaxf(na[q] - 2.0f * tau[q], 0.0f);
+                const float u1 = (t1 + 3.0f * kScrC * na[q]) * (1.0f + 3.0f * kScrC) + 1.0e-5f;
+                const float ru = __builtin_amdgcn_sqrtf(u1) * 1.000001f;
+                const float re = ru + screen_eps(fminf(big, (rna[q] + ru) * 1.001f), eps_floor);
+                th[q] = tau[q] > -inf ? 0.5f * (na[q] - near_limit(re, q)) : -3.0e38f;
+            }
+        }
+
+        // -- pass 2 ----------------------------------------------------------------------------------
+        int ch = 0, j = j0, evaluated = 0;
+        bool again = false;
+        while (ch < chunks && !tied) {
+            if (again) loadA();
+            again = true;
+            const int xs = 16 * NT * ch;
+            mask_cols(xs, th);
+            int queued = 0;
+            int found = 0;   // this lane's candidates in the queue
+            unsigned w[2];
+            walk(j, xs, [&](int jj, auto sc_, const scr_f4 (&acc)[NT]) {
+                constexpr int s = decltype(sc_)::value;
+                unsigned v = s & 1 ? w[s >> 1] : 0u;   // sign bits, shifted in: 1 where the candidate fails
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v = __builtin_amdgcn_alignbit(v, __float_as_uint(acc[t][q]), 31);
+                w[s >> 1] = v;
+                if constexpr (s == 3) {
+                    constexpr unsigned kAll = (1u << 8 * NT) - 1u;
+                    const unsigned w0 = ~w[0] & kAll, w1 = ~w[1] & kAll;
+                    found += __builtin_popcount(w0);
+                    found += __builtin_popcount(w1);
+                    const unsigned long long who = __ballot((w0 | w1) != 0u);
+                    const unsigned at = __builtin_amdgcn_mbcnt_hi((unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, (unsigned)queued));
+                    queue[(w0 | w1) != 0u ? at : (unsigned)G.queue] = vsz_u2{w0 | (unsigned)lane << 24, w1 | (unsigned)jj << 24};
+                    queued += __builtin_popcountll(who);
+                }
+            }, [&] { return j < j1 && queued <= G.queue - 64 && !__any(found > 24); });
+            if (j >= j1) {
+                ++ch;
+                j = j0;
+            }
+
+            // too many even before the first of them is evaluated?
+            const int all = wave_sum(found);
+            tied = evaluated + all > kScrMost;
+            if (tied) break;
+
+            // -- evaluate the queue, 8 lanes (columns) per candidate, 32 candidates at a time ----------
+            lds_order();
+            const int rf = lane >> 2, part = lane & 3;
+            // inserts the keys in kbuf: 4 lanes per block take a quarter each, then the lists merge
+            const auto insert = [&]() {
+                lds_order();
+                const int mine = min((int)ws->cnt[rf], kScrCap);
+                double L[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    L[k] = __builtin_bit_cast(double, part == 0 ? ws->best[rf * 8 + k] : kFill);
+                for (int k = part; k < mine; k += 4) key_insert(L, __builtin_bit_cast(double, ws->kbuf[rf * kScrCap + k]));
+                key_merge<kDppXor1>(L);
+                key_merge<kDppXor2>(L);
+                if (part == 0) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) ws->best[rf * 8 + k] = __builtin_bit_cast(unsigned long long, L[k]);
+                    ws->cnt[rf] = 0u;
+                }
+                lds_order();
+            };
+            const int corner = ry0 * S + rx0;
+            const unsigned corner_pos = (unsigned)(ry0 * 65536 + rx0);
+            int taken = 0;
+            unsigned w0 = 0u, w1 = 0u, from = 0u, group = 0u;   // an entry's candidates that are not listed yet
+            for (;;) {
+                // list candidates (block << 28 | row << 14 | column) in the space of the entries taken
+                int listed = 0;
+                for (;;) {
+                    const unsigned long long who = __ballot((w0 | w1) != 0u);
+                    const int more = __builtin_popcountll(who);
+                    if (more == 0) {
+                        if (taken >= queued) break;
+                        const vsz_u2 e = taken + lane < queued ? queue[taken + lane] : vsz_u2{0u, 0u};
+                        lds_order();
+                        w0 = e[0] & 0xffffffu;
+                        w1 = e[1] & 0xffffffu;
+                        from = e[0] >> 24;
+                        group = e[1] >> 24;
+                        taken += 64;
+                        continue;
+                    }
+                    if (listed + more > 2 * (taken < queued ? taken : G.queue)) break;
+                    if ((w0 | w1) != 0u) {
+                        const bool second = w0 == 0u;
+                        const unsigned w = second ? w1 : w0;
+                        const int top = __builtin_clz(w), o = top - (32 - 8 * NT);      // order of evaluation
+                        const unsigned rest = w & ~(0x80000000u >> top);
+                        w1 = second ? rest : w1;
+                        w0 = second ? 0u : rest;
+                        const int odd = o >= 4 * NT ? 1 : 0, tq = o - odd * 4 * NT;
+                        list[__builtin_amdgcn_mbcnt_hi((unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, (unsigned)listed))] =
+                            ((from >> 4) * 4u + (unsigned)(tq & 3)) << 28 | (4u * group + (second ? 2u : 0u) + (unsigned)odd) << 14 |
+                            ((unsigned)(xs + 16 * (tq >> 2)) + (from & 15u));
+                    }
+                    listed += more;
+                }
+                if (listed == 0) break;
+                lds_order();
+                // exact distances: 4 lanes a candidate, lane p + 2k with rows p, p + 2, .. of columns 4k..4k+3,
+                // 32 candidates at a time, the next ones' pixels in flight
+                struct Batch {
+                    unsigned bl[2], cp[2];
+                    vsz_u4 va[2][4], vb[2][4];
+                };
+                const int lane_off = ((lane & 1) * S + (lane & 2) * 2) * 4;
+                const auto fetch = [&](int f, Batch &b) {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const unsigned e = list[min(f + 16 * u + (lane >> 2), listed - 1)];
+                        const unsigned cy = e >> 14 & 0x3fffu, cx = e & 0x3fffu;
+                        b.bl[u] = e >> 28;
+                        b.cp[u] = corner_pos + (cy << 16) + cx;
+                        const unsigned rp = ws->refpos[b.bl[u]];
+                        const int oa = ((int)__umul24(pos_y(rp), S) + pos_x(rp)) * 4 + lane_off;
+                        const int ob = (corner + (int)__umul24(cy, S) + (int)cx) * 4 + lane_off;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            b.va[u][r] = __builtin_bit_cast(vsz_u4, __builtin_amdgcn_raw_buffer_load_b128(img.rsrc, oa, 2 * r * S * 4, 0));
+                            b.vb[u][r] = __builtin_bit_cast(vsz_u4, __builtin_amdgcn_raw_buffer_load_b128(img.rsrc, ob, 2 * r * S * 4, 0));
+                        }
+                    }
+                };
+                const auto evaluate = [&](int f, const Batch &b) {
+                    unsigned long long key[2];
+                    bool on[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // this lane's half of its columns
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) {
+                                const float d = __uint_as_float(b.va[u][r][c]) - __uint_as_float(b.vb[u][r][c]);
+                                e[c] = fmaf_(d, d, e[c]);
+                            }
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) e[c] += dpp_f<kDppXor1>(e[c]);
+                        float t = (e[0] + e[1]) + (e[2] + e[3]);
+                        t += dpp_f<kDppXor2>(t);
+                        t = t < FLT_MAX ? t : FLT_MAX;   // such a candidate never enters a list
+                        key[u] = (unsigned long long)__float_as_uint(t) << 32 | b.cp[u];
+                        on[u] = part == 0 && f + 16 * u + (lane >> 2) < listed && key[u] < ws->best[b.bl[u] * 8 + 7];
+                    }
+                    // where a block's buffer is full, its keys wait for an insertion
+                    for (;;) {
+                        bool over = false;
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            if (on[u]) {
+                                const unsigned slot = atomicAdd(&ws->cnt[b.bl[u]], 1u);
+                                if (slot < kScrCap) ws->kbuf[b.bl[u] * kScrCap + slot] = key[u];
+                                on[u] = slot >= kScrCap;
+                                over |= on[u];
+                            }
+                        if (!__any(over)) break;
+                        insert();
+                    }
+                };
+                Batch b0, b1;
+                fetch(0, b0);
+                for (int f = 0; f < listed; f += 64) {
+                    fetch(f + 32, b1);
+                    evaluate(f, b0);
+                    fetch(f + 64, b0);
+                    if (f + 32 < listed) evaluate(f + 32, b1);
+                }
+            }
+            insert();
+            evaluated += all;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                // with one chunk what follows are later rows: none enters a list of 8 zero distances
+                const float e7 = __uint_as_float((unsigned)(ws->best[(g * 4 + q) * 8 + 7] >> 32));
+                if (e7 == 0.0f && chunks == 1) th[q] = 3.0e38f;
+                else if (e7 < FLT_MAX) {
+                    const float lim = near_limit(__builtin_sqrtf(e7) * sc * 1.000002f, q);
+                    if (lim < FLT_MAX) th[q] = max_nan(th[q], 0.5f * (na[q] - lim));
+                }
+            }
+            lds_order();
+        }
+    } else if (flat) {
+        // a region of one value: every distance is 0, the list is the first 8 candidates in scan order
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int i = lane + 64 * u, k = i & 7;
+            const unsigned rp = ws->refpos[i >> 3];
+            const int xr = pos_x(rp), yr = pos_y(rp);
+            const int xa = max(xr - R, 0), nx = min(xr + R, W - 8) - xa + 1;
+            const int ya = max(yr - R, 0), ny = min(yr + R, H - 8) - ya + 1;
+            const int row = k / nx;
+            ws->best[i] = row < ny ? (unsigned long long)pack_xy(xa + k - row * nx, ya + row)
+                                   : (unsigned long long)__float_as_uint(FLT_MAX) << 32;
+        }
+    }
+    if (tied) {   // a third component of 1, which no list has, marks each block row of the tile
+        if (lane < 4 && bym + lane < a.nby) a.matches[((long long)(bym + lane) * a.nbx + bxm) * 8] = make_int4(0, 0, 1, 0);
+        return;
+    }
+    lds_order();
+
+    // self-inclusion (src/bm3d.cu:758-788), unless a temporal stage follows; then the lists, 16 bytes
+    // per lane
+    if (lane < 16 && !a.no_self) {
+        const unsigned self = ws->refpos[lane];
+        bool found = false;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) found |= (unsigned)ws->best[lane * 8 + k] == self;
+        if (!found) {
+#pragma unroll
+            for (int k = 7; k > 0; --k) ws->best[lane * 8 + k] = ws->best[lane * 8 + k - 1];
+            ws->best[lane * 8] = self;
+        }
+    }
+    lds_order();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = lane + 64 * u, rf = i >> 3;
+        const int bx = bxm + (rf & 3), by = bym + (rf >> 2);
+        const unsigned long long key = ws->best[i];
+        const unsigned pos = (unsigned)key;
+        if (bx < a.nbx && by < a.nby)
+            a.matches[((long long)by * a.nbx + bx) * 8 + (i & 7)] = make_int4(pos_x(pos), pos_y(pos), 0, (int)(key >> 32));
+    }
+}
+
+template <int NT>
+__global__ __launch_bounds__(64, 2) void k_match_screen(MatchArgs a, ScreenGeom G) {
+    extern __shared__ __align__(16) float region[];
+    match_screen_body<NT>(a, G, xcd_tile(blockIdx.x, gridDim.x), region);
+    zero_share(a);
+}
+
+// The tiles that the screen left: areas so even (letterbox bars after a first pass, graphics) that whole windows are
+// within its bounds, and tiles with non-finite values. Such tiles are few and the search waits for the longest, so
+// each is four workgroups, one per block row, and a wave searches one block: its lanes take half a search row
+// each in turn, from the region staged in LDS, and their lists merge as keys. VALU issue bounds a lane's
+// candidates, about 1100 cycles each. With one workgroup per tile and 16 lanes per block, a 128x96 frame with bars
+// took 131 us at block_step 4, bm_range 16, and 96 so (the scan alone: 178).
+__device__ __forceinline__ void match_tied_body(const MatchArgs &a, int LS, int tile, int row, float *region) {
+    const int lane = threadIdx.x & 63;
+    const int W = a.width, H = a.height, S = a.stride, bs = a.block_step, R = a.bm_range;
+    const int bxm = tile % a.tiles_x * 4, by = tile / a.tiles_x * 4 + row, bx = bxm + (int)(threadIdx.x >> 6);
+    const int y = min(min(by, a.nby - 1) * bs, H - 8), x = min(min(bx, a.nbx - 1) * bs, W - 8);
+    const int rx0 = min(bxm * bs, W - 8) - R, ry0 = y - R, RH = 2 * R + 8;
+    const int RW = min(min(bxm + 3, a.nbx - 1) * bs, W - 8) + R + 9 - rx0;   // (the scan loads a column ahead)
+    for (int Y = threadIdx.x >> 6; Y < RH; Y += 4)
+        for (int X = lane; X < RW; X += 64) {
+            const int gy = ry0 + Y, gx = rx0 + X;
+            region[lds_row(Y, LS) + X] = gy >= 0 && gy < H && gx >= 0 && gx < W ? a.img[(long long)gy * S + gx] : 0.0f;
+        }
+    __syncthreads();
+    if (bx < a.nbx && by < a.nby) {
+        RefPatch ref;
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) ref.a[r * 8 + c] = region[lds_row(R + r, LS) + x + c - rx0];
+        List8 L;
+        list_init<false>(L, 0);
+        for (int h = lane; h < 2 * (2 * R + 1); h += 64) {   // columns -R..-1 and 0..R of each row
+            const int dy = (h >> 1) - R, x0 = h & 1 ? x : x - R;
+            lds_scan<0>(region, LS, x0 - rx0, ry0, W, H, x0, y, h & 1 ? R : R - 1, dy, dy + 1, ref, L);
+        }
+        double K[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) K[k] = __builtin_bit_cast(double, (unsigned long long)__float_as_uint(L.er[k]) << 32 | L.pos[k]);
+        key_merge<kDppXor1>(K);
+        key_merge<kDppXor2>(K);
+        key_merge<kDppHalfMirror>(K);
+        key_merge<kDppMirror>(K);
+        for (int d = 16; d < 64; d *= 2) {
+            double o[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) o[k] = __shfl_xor(K[k], d);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) key_insert(K, o[k]);
+        }
+        unsigned long long out[8];
+        const unsigned self = pack_xy(x, y);
+        bool found = a.no_self != 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            out[k] = __builtin_bit_cast(unsigned long long, K[k]);
+            found |= (unsigned)out[k] == self;
+        }
+        if (!found) {
+#pragma unroll
+            for (int k = 7; k > 0; --k) out[k] = out[k - 1];
+            out[0] = self;
+        }
+        if (lane == 0) {
+            int4 *o = a.matches + ((long long)by * a.nbx + bx) * 8;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) o[k] = make_int4(pos_x((unsigned)out[k]), pos_y((unsigned)out[k]), 0, (int)(out[k] >> 32));
+        }
+    }
+    __syncthreads();   // the region before the next tile's
+}
+
+// Runs match_tied_body on the marked block rows of `tiles` tiles; plane(t, tile) gives a tile's arguments and its number
+// there.
+template <class Plane>
+__device__ __forceinline__ void match_tied(int tiles, int LS, float *region, const Plane &plane) {
+    __shared__ unsigned long long marked[4];
+    const int per = gridDim.x;
+    for (int u0 = blockIdx.x; u0 < 4 * tiles; u0 += 256 * per) {
+        const int u = u0 + (int)threadIdx.x * per;   // neighbours go to different workgroups
+        bool on = false;
+        if (u < 4 * tiles) {
+            int tile;
+            const MatchArgs &a = plane(u >> 2, tile);
+            const int by = tile / a.tiles_x * 4 + (u & 3);
+            on = by < a.nby && a.matches[((long long)by * a.nbx + tile % a.tiles_x * 4) * 8].z == 1;
+        }
+        const unsigned long long who = __ballot(on);
+        if ((threadIdx.x & 63) == 0) marked[threadIdx.x >> 6] = who;
+        __syncthreads();
+        for (int w = 0; w < 4; ++w)
+            for (unsigned long long m = marked[w]; m; m &= m - 1) {
+                const int v = u0 + (64 * w + __builtin_ctzll(m)) * per;
+                int tile;
+                const MatchArgs &a = plane(v >> 2, tile);
+                match_tied_body(a, LS, tile, v & 3, region);
+            }
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(256) void k_match_tied(MatchArgs a, int tiles, int LS) {
+    extern __shared__ __align__(16) float region[];
+    match_tied(tiles, LS, region, [&](int t, int &tile) -> const MatchArgs & {
+        tile = t;
+        return a;
+    });
+}
+
 // Spatial search on raw buffer loads, for windows whose staged region exceeds the LDS budget: one
 // lane per reference block, 8 x 8 blocks per wave.
 template <int M>
@@ -1022,11 +1974,6 @@ __global__ __launch_bounds__(64, 2) void k_match_temporal(MatchArgs a) {
 // switch is an 8x8 transpose per rank through a per-group LDS buffer. LDS instructions of one
 // wave execute in order, so the transposes only need compiler barriers, not waits.
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ void lds_order() {
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
-}
-
 // Switches all 8 ranks between column and row layout (the transpose is its own inverse).
 __device__ __forceinline__ void transpose_ranks(float *v, float *buf, int l8) {
 #pragma unroll
@@ -1068,7 +2015,6 @@ struct SplitOp {
 
 typedef __bf16 vsz_b2 __attribute__((ext_vector_type(2)));
 typedef float vsz_f2 __attribute__((ext_vector_type(2)));
-typedef unsigned vsz_u2 __attribute__((ext_vector_type(2)));
 
 // Two floats rounded to bf16 (round to nearest even), packed: one v_cvt_pk_bf16_f32.
 __device__ __forceinline__ unsigned pk_bf16(float a, float b) {
@@ -1947,6 +2893,26 @@ __global__ __launch_bounds__(256) void k_match_lds4_batch(const BatchTable *__re
     zero_range(zero, zero_n64);
 }
 
+template <int NT>
+__global__ __launch_bounds__(64, 2) void k_match_screen_batch(const BatchTable *__restrict__ t, ScreenGeom G,
+                                                              unsigned long long *zero, long long zero_n64) {
+    extern __shared__ __align__(16) float region[];
+    const int g = xcd_tile(blockIdx.x, gridDim.x);
+    const int p = batch_plane(t->match_off, t->n, g);
+    const MatchArgs &a = t->m[p];
+    match_screen_body<NT>(a, G, g - t->match_off[p], region);
+    zero_range(zero, zero_n64);
+}
+
+__global__ __launch_bounds__(256) void k_match_tied_batch(const BatchTable *__restrict__ tab, int tiles, int LS) {
+    extern __shared__ __align__(16) float region[];
+    match_tied(tiles, LS, region, [&](int t, int &tile) -> const MatchArgs & {
+        const int p = batch_plane(tab->match_off, tab->n, t);
+        tile = t - tab->match_off[p];
+        return tab->m[p];
+    });
+}
+
 template <bool FINAL, int T2, int T1, bool EXACT>
 __global__ __launch_bounds__(256, T2 == kDctMfma ? 4 : 2) void k_filter_tile_batch(const BatchTable *__restrict__ t) {
     extern __shared__ float smem[];
@@ -2180,6 +3146,7 @@ Layout layout_of(const vsz_bm3d_kparams *p) {
 // LDS bytes the staged matcher needs for a full 16 x 8*WR block tile (0: does not fit).
 constexpr size_t kMatchLdsBudget = 80 * 1024;  // two 256-lane workgroups per CU
 
+
 size_t match_lds_bytes(int block_step, int bm_range, int *lds_stride, int wr = 2, int split = 1) {
     const long long rw = 15LL * block_step + 2LL * bm_range + 9;
     const long long rh = (8LL * wr / split - 1) * block_step + 2LL * bm_range + 8;
@@ -2202,6 +3169,40 @@ size_t match_lds4_bytes(const MatchArgs &a, int *lds_stride) {
 
 // Which kernel runs a spatial (or centre-frame) search.
 enum MatchKernel { kMkLds4 = 0, kMkLds1, kMkLds2, kMkLds4Bands, kMkLdsShort, kMkGlobal };
+
+// k_match_tied: row pitch (odd, the lanes of a block read rows a constant apart; lds_row shifts rows by up to 3) and bytes of its staged region, at most
+// 30 KB where the screen runs; workgroups, which share out the marked block rows.
+int tied_pitch(int bs, int R) { return (3 * bs + 2 * R + 12) | 1; }
+size_t tied_lds_bytes(int bs, int R) { return ((size_t)(2 * R + 8) * tied_pitch(bs, R) + 3) * 4; }
+int tied_wgs(int tiles) { return (int)std::min(4LL * tiles, 1024LL); }
+
+// Columns per product pass of the screened search: tiles of 16 in sets of two or three, whichever leaves
+// fewer.
+int screen_nt(int bs, int R) {
+    return screen_geom(bs, R, 2).tiles < screen_geom(bs, R, 3).tiles ? 2 : 3;
+}
+
+ScreenGeom screen_plan(int bs, int R) { return screen_geom(bs, R, screen_nt(bs, R)); }
+
+// Whether the screened search takes a spatial ssd search of so many 4 x 4 block tiles. Its cost per block hardly
+// depends on the window below 48 columns, the scan's grows with its area. Times of whole passes (scan / screened, us, frames
+// with noise and the same with letterbox bars, whose tiles are searched twice):
+//   tiles   240: bm_range 8 71/59 and 71/70, 9 77/60 and 76/70, 16 157/81 and 158/109 (640x360, block_step 8)
+//   tiles   920: bm_range 8 97/94 and 97/105, 9 106/97 and 104/107, 12 136/115 and 135/131, 16 179/113 and 179/146
+//   tiles  8160: bm_range 9 251/227 and 244/251, 12 336/263 and 330/302, 16 477/278 and 473/361 (1920x1080, block_step 4)
+// so it starts at 8 where one wave per SIMD takes all tiles and at 12 elsewhere; at 16 where its region exceeds an
+// eighth of a CU's LDS (block_step 8: 12 170/175 and 165/195, 16 229/184 and 224/231 at 1920x1080). Above a quarter
+// (bm_range 24 at block_step 8) it no longer gains.
+bool screen_fits(int bs, int R) { return R < 1024 && screen_lds_bytes(screen_plan(bs, R)) <= kScrLdsMax; }
+
+bool screen_pays(int bs, int R, long long tiles) {
+    if (!screen_fits(bs, R)) return false;
+    return R >= (tiles <= 512 ? 8 : screen_lds_bytes(screen_plan(bs, R)) <= kScrLds8 ? 12 : 16);
+}
+
+bool screened(const MatchArgs &a, int metric) {
+    return metric == 0 && screen_pays(a.block_step, a.bm_range, (long long)((a.nbx + 3) / 4) * ((a.nby + 3) / 4));
+}
 
 struct MatchPlan {
     MatchKernel kernel;
@@ -2241,6 +3242,17 @@ MatchPlan plan_match(const MatchArgs &a, int metric) {
 
 template <int M> void launch_spatial(const MatchArgs &a, const MatchPlan &pl, hipStream_t s) {
     MatchArgs b = a;
+    if (screened(a, M)) {
+        const ScreenGeom G = screen_plan(a.block_step, a.bm_range);
+        const size_t lds = screen_lds_bytes(G);
+        b.tiles_x = (a.nbx + 3) / 4;
+        const dim3 grid((unsigned)(b.tiles_x * ((a.nby + 3) / 4)));
+        if (screen_nt(a.block_step, a.bm_range) == 2) hipLaunchKernelGGL(k_match_screen<2>, grid, dim3(64), lds, s, b, G);
+        else hipLaunchKernelGGL(k_match_screen<3>, grid, dim3(64), lds, s, b, G);
+        hipLaunchKernelGGL(k_match_tied, dim3(tied_wgs((int)grid.x)), dim3(256), tied_lds_bytes(a.block_step, a.bm_range), s, b,
+                           (int)grid.x, tied_pitch(a.block_step, a.bm_range));
+        return;
+    }
     b.lds_stride = pl.lds_stride;
     switch (pl.kernel) {
     case kMkLds4:
@@ -2807,6 +3819,15 @@ void launch_match_batch(int metric, bool shared_cols, const BatchTable *d, int w
     }
 }
 
+void launch_match_screen_batch(int bs, int R, const BatchTable *d, int wgs, unsigned long long *zero, long long n64,
+                               hipStream_t s) {
+    const ScreenGeom G = screen_plan(bs, R);
+    const size_t lds = screen_lds_bytes(G);
+    if (screen_nt(bs, R) == 2) hipLaunchKernelGGL(k_match_screen_batch<2>, dim3(wgs), dim3(64), lds, s, d, G, zero, n64);
+    else hipLaunchKernelGGL(k_match_screen_batch<3>, dim3(wgs), dim3(64), lds, s, d, G, zero, n64);
+    hipLaunchKernelGGL(k_match_tied_batch, dim3(tied_wgs(wgs)), dim3(256), tied_lds_bytes(bs, R), s, d, wgs, tied_pitch(bs, R));
+}
+
 void launch_match_global_batch(int metric, const BatchTable *d, int wgs, unsigned long long *zero, long long n64,
                                hipStream_t s) {
     switch (metric) {
@@ -2873,6 +3894,7 @@ struct vsz_bm3d_batch {
     bool shared_cols = false;  // every plane takes the shared-column block_step-4 matcher
     bool sc_allowed = false;   // ... may take it (the autotuner then times both matchers)
     bool global_match = false;  // windows beyond the LDS matchers' budget: the global-memory matcher
+    bool screen_ok = false;     // the staged schedule searches with the screened kernel (as `screened` for one plane)
     bool direct_filter = false; // a region beyond the filter tiles' LDS budget: direct-atomic filtering
     size_t lds_rows = 0, lds_sc = 0;
     int stride_rows = 0, stride_sc = 0;
@@ -2924,10 +3946,13 @@ struct vsz_bm3d_batch {
             for (const auto &pl : planes) m = std::max(m, pl.tile[pass].lds_bytes);
         return m;
     }
+    bool screen() const { return screen_ok && schedule == VSZ_BATCH_STAGED; }
     int match_tiles_x(const BatchPlane &pl) const {
+        if (screen()) return (pl.L.nbx + 3) / 4;
         return global_match ? (pl.L.nbx + 7) / 8 : shared_cols ? (pl.L.nbx + 14) / 15 : (pl.L.nbx + 15) / 16;
     }
     int match_tiles_y(const BatchPlane &pl) const {
+        if (screen()) return (pl.L.nby + 3) / 4;
         return global_match ? (pl.L.nby + 7) / 8 : shared_cols ? (pl.L.nby + 7) / 8 : (pl.L.nby + 15) / 16;
     }
     // workgroups of one plane's matching (the global matcher: four 8 x 8-block tiles each)
@@ -3037,6 +4062,7 @@ struct vsz_bm3d_batch {
             const BatchTable *d = d_tab + pass;
             unsigned long long *acc = (unsigned long long *)(work + pass * acc_span);
             if (global_match) launch_match_global_batch(bp.metric, d, match_wgs(), acc, n64, s);
+            else if (screen()) launch_match_screen_batch(bp.block_step, bp.bm_range, d, match_wgs(), acc, n64, s);
             else launch_match_batch(bp.metric, shared_cols, d, match_wgs(), match_lds, acc, n64, s);
             const int fw = filter_wgs(pass);
             const size_t fl = filter_lds(pass);
@@ -3320,6 +4346,7 @@ int vsz_bm3d_batch_create(const vsz_bm3d_batch_params *bp, const vsz_bm3d_plane 
         b->sc_allowed = b->lds_sc != 0;
     }
     b->global_match = !b->lds_rows && !b->sc_allowed;  // windows beyond the LDS matchers' budget
+    b->screen_ok = bp->metric == 0 && !b->global_match && screen_pays(bp->block_step, bp->bm_range, LLONG_MAX);
     b->use_matcher(b->sc_allowed);
     const float fac[2] = {bits_float(0x3f021bb6u), bits_float(0x3e40c0c1u)};  // src/bm3d.zig:1013-1024
     size_t acc = 0, rest = 0;

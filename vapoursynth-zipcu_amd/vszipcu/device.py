@@ -66,7 +66,7 @@ def num_blocks(p: _lib.KParams):
 
 
 def match_plan(p: _lib.KParams) -> str:
-    """Name of the matcher vsz_bm3d_match launches for these parameters (no GPU needed)."""
+    """Name of the exhaustive matcher of vsz_bm3d_match for these parameters (no GPU needed)."""
     name = _lib.load().vsz_bm3d_match_plan(C.byref(p)).decode()
     if not name:
         raise RuntimeError(f"vszipcu: {_lib.last_error()}")
