@@ -152,16 +152,33 @@ __global__ __launch_bounds__(256) void k_conv3x3(const unsigned short *__restric
 // Weight gradient dW[t][out][in] += sum over pixels of dy[p][out] * x[p + t][in], FP32.
 // A workgroup walks `tiles` consecutive 16x16 tiles (row-major over images) accumulating in
 // registers, then adds its partial sums with device atomics. Wave w owns the (out half, in half)
-// pair w for all 9 taps. LDS holds dy transposed ([out][16 rows][16 cols]) and x transposed in
-// three horizontally shifted copies ([dx][in][18 rows][16 cols]) so every MFMA operand is 16
-// aligned bytes.
+// pair w for all 9 taps. LDS holds dy ([out][16 rows][16 cols]) and the halo of x ([in][18 rows][18 cols])
+// transposed. A wave reads 10 columns of a halo row and makes the operands of the row's three taps
+// from them by shifting, so x is stored once; pixels are transposed in pairs, one 32-bit store
+// per channel. The next tile's pixels are loaded into registers during the current one's products.
+// Bound by latency at one workgroup per CU and by the atomics at its end (the products take 5 us of
+// 32x128x128 pixels, its 67 MB 14 us at copy speed): 63 us with three shifted copies of x, stored 16 bits at a time, and
+// no loads ahead; 34 now.
 constexpr int DY_CH_BYTES = TILE * TILE * 2 + 16;       // 528
-constexpr int XS_CH_BYTES = HALO * TILE * 2 + 16;        // 592
+constexpr int XS_ROW = HALO / 2;                         // dwords of a halo row
+constexpr int XS_CH = HALO * XS_ROW + 1;                 // ... of a channel; odd: channels start in different banks
+constexpr int kXPairs = HALO * XS_ROW * 4, kXPer = (kXPairs + 255) / 256;   // 16-byte parts of pixel pairs
+constexpr int kDyPairs = TILE * TILE / 2 * 4, kDyPer = kDyPairs / 256;
 
-__global__ __launch_bounds__(256) void k_conv3x3_dw(const unsigned short *__restrict__ x, const unsigned short *__restrict__ dy,
-                                                    int N, int H, int W, int tiles, float *__restrict__ dw) {
+// The 16-bit values of two pixels' 8 channels as 8 (first, second) dwords at lds[0], lds[stride], ..
+__device__ __forceinline__ void store_pair(unsigned *lds, int stride, const uint4 &a, const uint4 &b) {
+    const unsigned p[4] = {a.x, a.y, a.z, a.w}, q[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        lds[(2 * k) * stride] = __builtin_amdgcn_perm(q[k], p[k], 0x05040100u);
+        lds[(2 * k + 1) * stride] = __builtin_amdgcn_perm(q[k], p[k], 0x07060302u);
+    }
+}
+
+__global__ __launch_bounds__(256, 2) void k_conv3x3_dw(const unsigned short *__restrict__ x, const unsigned short *__restrict__ dy,
+                                                       int N, int H, int W, int tiles, float *__restrict__ dw) {
     __shared__ __attribute__((aligned(16))) char sdy[CH * DY_CH_BYTES];
-    __shared__ __attribute__((aligned(16))) char sx[3 * CH * XS_CH_BYTES];
+    __shared__ unsigned sx[CH * XS_CH];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane & 15, g = lane >> 4;
     const int oh = wave >> 1, ih = wave & 1;
@@ -172,43 +189,48 @@ __global__ __launch_bounds__(256) void k_conv3x3_dw(const unsigned short *__rest
 #pragma unroll
     for (int t = 0; t < 9; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    for (int k = 0; k < tiles; ++k) {
-        const int tile = blockIdx.x * tiles + k;
-        if (tile >= total) break;
+    uint4 vd[kDyPer][2], vx[kXPer][2];
+    // pixels outside the image are zero
+    const auto pixel = [&](const unsigned short *src, int n, int gy, int gx, int part) {
+        return gy >= 0 && gy < H && gx >= 0 && gx < W
+                   ? *reinterpret_cast<const uint4 *>(src + (((long long)n * H + gy) * W + gx) * CH + part * 8)
+                   : make_uint4(0, 0, 0, 0);
+    };
+    const auto load = [&](int tile) {
         const int n = tile / (tx_n * ty_n), rem = tile % (tx_n * ty_n);
         const int x0 = (rem % tx_n) * TILE, y0 = (rem / tx_n) * TILE;
-        __syncthreads();  // previous tile's LDS reads are done
-        // dy tile, transposed; pixels outside the image contribute zero
-        for (int i = threadIdx.x; i < TILE * TILE * 4; i += 256) {
-            const int pix = i >> 2, part = i & 3;
-            const int ry = pix / TILE, rx = pix % TILE;
-            const int gy = y0 + ry, gx = x0 + rx;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (gy < H && gx < W) v = *reinterpret_cast<const uint4 *>(dy + (((long long)n * H + gy) * W + gx) * CH + part * 8);
-            const unsigned short *e = reinterpret_cast<const unsigned short *>(&v);
 #pragma unroll
-            for (int c = 0; c < 8; ++c)
-                *reinterpret_cast<unsigned short *>(sdy + (part * 8 + c) * DY_CH_BYTES + (ry * TILE + rx) * 2) = e[c];
+        for (int k = 0; k < kDyPer; ++k) {
+            const int i = (int)threadIdx.x + 256 * k, pair = i >> 2;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                vd[k][e] = pixel(dy, n, y0 + pair / (TILE / 2), x0 + pair % (TILE / 2) * 2 + e, i & 3);
         }
-        // x halo rows -1..16, copies for dx = -1, 0, +1
-        for (int i = threadIdx.x; i < HALO * HALO * 4; i += 256) {
-            const int pix = i >> 2, part = i & 3;
-            const int hy = pix / HALO, hx = pix % HALO;  // halo coordinates: gx = x0 + hx - 1
-            const int gy = y0 + hy - 1, gx = x0 + hx - 1;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (gy >= 0 && gy < H && gx >= 0 && gx < W)
-                v = *reinterpret_cast<const uint4 *>(x + (((long long)n * H + gy) * W + gx) * CH + part * 8);
-            const unsigned short *e = reinterpret_cast<const unsigned short *>(&v);
 #pragma unroll
-            for (int s = 0; s < 3; ++s) {  // copy s holds column c = hx - s (dx = s - 1)
-                const int c = hx - s;
-                if (c < 0 || c >= TILE) continue;
+        for (int k = 0; k < kXPer; ++k) {
+            const int i = (int)threadIdx.x + 256 * k, pair = i >> 2;
+            if (i < kXPairs)
 #pragma unroll
-                for (int q = 0; q < 8; ++q)
-                    *reinterpret_cast<unsigned short *>(sx + (s * CH + part * 8 + q) * XS_CH_BYTES + (hy * TILE + c) * 2) = e[q];
-            }
+                for (int e = 0; e < 2; ++e)
+                    vx[k][e] = pixel(x, n, y0 + pair / XS_ROW - 1, x0 + pair % XS_ROW * 2 + e - 1, i & 3);
+        }
+    };
+    const int first = blockIdx.x * tiles, last = min(first + tiles, total);
+    if (first < last) load(first);
+    for (int tile = first; tile < last; ++tile) {
+        __syncthreads();  // previous tile's LDS reads are done
+#pragma unroll
+        for (int k = 0; k < kDyPer; ++k) {
+            const int i = (int)threadIdx.x + 256 * k;
+            store_pair(reinterpret_cast<unsigned *>(sdy + (i & 3) * 8 * DY_CH_BYTES) + (i >> 2), DY_CH_BYTES / 4, vd[k][0], vd[k][1]);
+        }
+#pragma unroll
+        for (int k = 0; k < kXPer; ++k) {
+            const int i = (int)threadIdx.x + 256 * k;
+            if (i < kXPairs) store_pair(sx + (i & 3) * 8 * XS_CH + (i >> 2), XS_CH, vx[k][0], vx[k][1]);
         }
         __syncthreads();
+        if (tile + 1 < last) load(tile + 1);
         // K = 256 pixels in 8 chunks of 32: chunk c = rows 2c, 2c+1; lane group g takes row
         // 2c + (g >> 1), columns 8*(g & 1)..+7
 #pragma unroll
@@ -216,11 +238,18 @@ __global__ __launch_bounds__(256) void k_conv3x3_dw(const unsigned short *__rest
             const int ry = 2 * c + (g >> 1), cx = 8 * (g & 1);
             const bf16x8 a = *reinterpret_cast<const bf16x8 *>(sdy + (oh * 16 + j) * DY_CH_BYTES + (ry * TILE + cx) * 2);
 #pragma unroll
-            for (int t = 0; t < 9; ++t) {
-                const int ky = t / 3, kx = t % 3;  // x row = ry + ky - 1 -> halo row ry + ky
-                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(sx + (kx * CH + ih * 16 + j) * XS_CH_BYTES +
-                                                                   ((ry + ky) * TILE + cx) * 2);
-                acc[t] = mfma(a, b, acc[t]);
+            for (int ky = 0; ky < 3; ++ky) {  // x row = ry + ky - 1 -> halo row ry + ky, columns cx + kx
+                const unsigned *p = sx + (ih * 16 + j) * XS_CH + (ry + ky) * XS_ROW + cx / 2;
+                unsigned d[5], m[4];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) d[k] = p[k];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) m[k] = __builtin_amdgcn_alignbit(d[k + 1], d[k], 16);
+                const uint4 b0 = make_uint4(d[0], d[1], d[2], d[3]), b1 = make_uint4(m[0], m[1], m[2], m[3]);
+                const uint4 b2 = make_uint4(d[1], d[2], d[3], d[4]);
+                acc[3 * ky] = mfma(a, __builtin_bit_cast(bf16x8, b0), acc[3 * ky]);
+                acc[3 * ky + 1] = mfma(a, __builtin_bit_cast(bf16x8, b1), acc[3 * ky + 1]);
+                acc[3 * ky + 2] = mfma(a, __builtin_bit_cast(bf16x8, b2), acc[3 * ky + 2]);
             }
         }
     }
@@ -231,19 +260,42 @@ __global__ __launch_bounds__(256) void k_conv3x3_dw(const unsigned short *__rest
         for (int q = 0; q < 4; ++q) atomicAdd(dw + (t * CH + oh * 16 + g * 4 + q) * CH + ih * 16 + j, acc[t][q]);
 }
 
-// db[out] += sum over pixels of dy[p][out].
-__global__ __launch_bounds__(256) void k_bias_grad(const unsigned short *__restrict__ dy, long long pixels, float *__restrict__ db) {
-    __shared__ float part[8][CH];
-    const int c = threadIdx.x & 31, r = threadIdx.x >> 5;
-    float s = 0.0f;
-    for (long long p = (long long)blockIdx.x * 8 + r; p < pixels; p += (long long)gridDim.x * 8) s += bf2f(dy[p * CH + c]);
-    part[r][c] = s;
-    __syncthreads();
-    if (r == 0) {
-        float t = 0.0f;
-        for (int k = 0; k < 8; ++k) t += part[k][c];
-        atomicAdd(db + c, t);
+// db[out] += sum over pixels of dy[p][out]. A lane adds 8 channels of every 64th pixel of its workgroup's
+// share, 8 loads of 16 bytes in flight. Bound by the read; 32x128x128 pixels (34 MB): 63 us with
+// 2-byte loads one after another, 8.6 now.
+__global__ __launch_bounds__(256) void k_bias_grad(const unsigned short *__restrict__ dy, long long pixels, long long share,
+                                                   float *__restrict__ db) {
+    constexpr int kAhead = 8;
+    __shared__ float part[4][CH];
+    const int c = threadIdx.x & 3;
+    const long long first = blockIdx.x * share, last = first + share < pixels ? first + share : pixels;
+    float s[8] = {};
+    for (long long p = first + (threadIdx.x >> 2); p < last; p += 64 * kAhead) {
+        uint4 v[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k)
+            v[k] = p + 64 * k < last ? *reinterpret_cast<const uint4 *>(dy + (p + 64 * k) * CH + c * 8) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const unsigned u[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                s[2 * q] += __uint_as_float(u[q] << 16);
+                s[2 * q + 1] += __uint_as_float(u[q] & 0xffff0000u);
+            }
+        }
     }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+#pragma unroll
+        for (int o = 4; o < 64; o <<= 1) s[q] += __shfl_xor(s[q], o);
+    }
+    if ((threadIdx.x & 63) < 4)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) part[threadIdx.x >> 6][c * 8 + q] = s[q];
+    __syncthreads();
+    if (threadIdx.x < CH)
+        atomicAdd(db + threadIdx.x, (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]));
 }
 
 // x0[n][y][x] = (noisy, sigma_map, 0 ... 0) as bf16; noisy is fp32 [N][H][stride].
@@ -265,24 +317,28 @@ __global__ __launch_bounds__(256) void k_pack_input(const float *__restrict__ no
 }
 
 // Mean squared error against `target`; writes the output-layer gradient (channel 0 of a
-// [N][H][W][32] bf16 tensor, the rest zero) and accumulates the loss sum.
+// [N][H][W][32] bf16 tensor, the rest zero) and accumulates the loss sum. Four lanes per pixel store 16 bytes
+// each, consecutive lanes consecutive bytes. Each workgroup adds to the loss once: additions to one address take
+// 13 ns apiece, and one per wave was most of the time (32x128x128 pixels: 109 us, 18 now).
 __global__ __launch_bounds__(256) void k_loss_grad(const float *__restrict__ out, const float *__restrict__ target,
                                                    long long pixels, float scale, unsigned short *__restrict__ g,
                                                    float *__restrict__ loss) {
-    const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
-    float d = 0.0f;
-    if (p < pixels) {
-        d = out[p] - target[p];
-        __bf16 h[8] = {(__bf16)(2.0f * scale * d), (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f,
-                       (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f};
-        uint4 *dst = reinterpret_cast<uint4 *>(g + p * CH);
-        dst[0] = *reinterpret_cast<const uint4 *>(h);
-        dst[1] = dst[2] = dst[3] = make_uint4(0, 0, 0, 0);
+    __shared__ float part[4];
+    const int c = threadIdx.x & 3;
+    float s = 0.0f;
+    for (long long p = (long long)blockIdx.x * 64 + (threadIdx.x >> 2); p < pixels; p += (long long)gridDim.x * 64) {
+        const float d = out[p] - target[p];
+        const __bf16 h = (__bf16)(2.0f * scale * d);
+        const unsigned lo = __builtin_bit_cast(unsigned short, h);
+        reinterpret_cast<uint4 *>(g + p * CH)[c] = make_uint4(c == 0 ? lo : 0u, 0, 0, 0);
+        s += d * d;
     }
-    float s = d * d;
+    s = c == 0 ? s : 0.0f;   // the four lanes of a pixel hold the same
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if ((threadIdx.x & 63) == 0) atomicAdd(loss, s * scale);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(loss, ((part[0] + part[1]) + (part[2] + part[3])) * scale);
 }
 
 // Adam on the fp32 master parameters, then the bf16 copies: forward layout w[t][o][i] and the
@@ -448,6 +504,11 @@ __global__ __launch_bounds__(256) void k_end_weights(const unsigned short *__res
 using namespace vszcnn;
 
 namespace {
+// Workgroups of the reductions, at most: each ends in device atomics on the same few addresses, which twice as
+// many make the longer part (32x128x128 pixels: weight gradient 34 us, 41 with 512; bias gradient 8.6 and 11.7; loss 18
+// and 21 with 1024).
+constexpr long long kDwGroups = 256, kBiasGroups = 256, kLossGroups = 512;
+
 int launch_ok(const char *what) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return vsz_fail(VSZ_EDEVICE, "%s: %s", what, hipGetErrorString(e));
@@ -511,7 +572,7 @@ int vsz_cnn_run(const vsz_cnn_model *m, const float *noisy, int n, int h, int wd
 int vsz_cnn_conv3x3_dw(const void *x, const void *dy, int n, int h, int wd, float *dw, void *stream) {
     if (!x || !dy || !dw || n < 1 || h < 1 || wd < 1) return vsz_fail(VSZ_EINVAL, "vsz_cnn_conv3x3_dw: invalid arguments");
     const long long total = (long long)n * ((wd + TILE - 1) / TILE) * ((h + TILE - 1) / TILE);
-    const int tiles = 8;
+    const int tiles = (int)((total + kDwGroups - 1) / kDwGroups);
     const unsigned grid = (unsigned)((total + tiles - 1) / tiles);
     hipLaunchKernelGGL(k_conv3x3_dw, dim3(grid), dim3(256), 0, (hipStream_t)stream, (const unsigned short *)x,
                        (const unsigned short *)dy, n, h, wd, tiles, dw);
@@ -520,8 +581,9 @@ int vsz_cnn_conv3x3_dw(const void *x, const void *dy, int n, int h, int wd, floa
 
 int vsz_cnn_bias_grad(const void *dy, long long pixels, float *db, void *stream) {
     if (!dy || !db || pixels < 1) return vsz_fail(VSZ_EINVAL, "vsz_cnn_bias_grad: invalid arguments");
-    const unsigned grid = (unsigned)std::min<long long>((pixels + 2047) / 2048, 1024);
-    hipLaunchKernelGGL(k_bias_grad, dim3(grid), dim3(256), 0, (hipStream_t)stream, (const unsigned short *)dy, pixels, db);
+    const long long share = std::max<long long>(512, ((pixels + kBiasGroups - 1) / kBiasGroups + 63) / 64 * 64);
+    hipLaunchKernelGGL(k_bias_grad, dim3((unsigned)((pixels + share - 1) / share)), dim3(256), 0, (hipStream_t)stream,
+                       (const unsigned short *)dy, pixels, share, db);
     return launch_ok("vsz_cnn_bias_grad");
 }
 
@@ -537,7 +599,7 @@ int vsz_cnn_pack_input(const float *noisy, int n, int h, int wd, int stride, con
 
 int vsz_cnn_loss_grad(const float *out, const float *target, long long pixels, void *grad, float *loss, void *stream) {
     if (!out || !target || !grad || !loss || pixels < 1) return vsz_fail(VSZ_EINVAL, "vsz_cnn_loss_grad: invalid arguments");
-    hipLaunchKernelGGL(k_loss_grad, dim3((unsigned)((pixels + 255) / 256)), dim3(256), 0, (hipStream_t)stream, out, target,
+    hipLaunchKernelGGL(k_loss_grad, dim3((unsigned)std::min<long long>((pixels + 63) / 64, kLossGroups)), dim3(256), 0, (hipStream_t)stream, out, target,
                        pixels, 1.0f / (float)pixels, (unsigned short *)grad, loss);
     return launch_ok("vsz_cnn_loss_grad");
 }
