@@ -79,8 +79,13 @@ __device__ __forceinline__ void stage_halo(const unsigned short *x, int n, int H
 //   2: acc * (aux[n][y][x][out] > 0) -> bf16 (backward data through the previous ReLU)
 // Persistent: workgroup g walks the 16x16 tiles g, g + G, ... (row-major over images) and loads
 // the next tile's halo into registers while it computes the current one from LDS; the weights
-// are loaded once. Wave w computes output channels hh*16 .. +15 (hh = w & 1) of rows
-// (w >> 1)*8 .. +7 of a tile.
+// are loaded once. Wave w computes rows 4w .. 4w+3 of a tile, all 32 output channels and all rows at once,
+// from one read of each pixel of the halo: eight sums in flight, a quarter of the LDS reads of one row and 16 channels at
+// a time. Row 4g + q of product h is channel 8g + 4h + q, so a lane ends
+// with 8 consecutive channels of a pixel and stores 16 bytes, a wave 1 KB in a row.
+// Bound by memory (3x1920x1080: 796 MB, 163 us at copy speed; 192 us measured). The estimate of three such frames, four
+// of these layers of six, took 925 us with a row and 16 channels at a time (8-byte stores), 885 with a row and
+// 32 channels and 878 so; the training step 576, 558 and 554. Unrolled it takes 212 VGPRs: two workgroups per CU.
 __global__ __launch_bounds__(256) void k_conv3x3(const unsigned short *__restrict__ x, const unsigned short *__restrict__ w,
                                                  const float *__restrict__ bias, int N, int H, int W, int tiles, int mode,
                                                  const unsigned short *__restrict__ aux, const float *__restrict__ base,
@@ -89,16 +94,17 @@ __global__ __launch_bounds__(256) void k_conv3x3(const unsigned short *__restric
     const int tx_n = (W + TILE - 1) / TILE, ty_n = (H + TILE - 1) / TILE;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane & 15, g = lane >> 4;
-    const int hh = wave & 1, r0 = (wave >> 1) * 8;
-    const bool active = !(mode == 1 && hh == 1);  // the residual output layer needs output channel 0 only
-    bf16x8 wa[9];
+    const int r0 = wave * 4, o = g * 8;
+    bf16x8 wa[2][9];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) wa[t] = *reinterpret_cast<const bf16x8 *>(w + ((t * CH) + hh * 16 + j) * CH + g * 8);
-    const int o = hh * 16 + g * 4;
-    float bo[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+            wa[h][t] = *reinterpret_cast<const bf16x8 *>(w + ((t * CH) + (j >> 2) * 8 + h * 4 + (j & 3)) * CH + g * 8);
+    float bo[8] = {};
     if (mode != 2)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) bo[q] = bias[mode == 1 ? 0 : o + q];
+        for (int q = 0; q < 8; ++q) bo[q] = bias[mode == 1 ? 0 : o + q];
 
     uint4 v[kHaloPer];
     int tile = blockIdx.x;
@@ -110,41 +116,52 @@ __global__ __launch_bounds__(256) void k_conv3x3(const unsigned short *__restric
         __syncthreads();
         const int nt = tile + gridDim.x;
         if (nt < tiles) halo_load(x, nt / (tx_n * ty_n), H, W, (nt % tx_n) * TILE, ((nt / tx_n) % ty_n) * TILE, v);
-        if (!active) continue;
-#pragma unroll 2
-        for (int rr = 0; rr < 8; ++rr) {
-            const int r = r0 + rr;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        f32x4 acc[4][2];
 #pragma unroll
-            for (int t = 0; t < 9; ++t) {
-                const int ky = t / 3, kx = t % 3;
-                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(lds + ((r + ky) * HALO + j + kx) * PIX_BYTES + g * 16);
-                acc = mfma(wa[t], b, acc);
+        for (int rr = 0; rr < 4; ++rr) acc[rr][0] = acc[rr][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // a halo row's pixels are read once for the three rows that they meet
+#pragma unroll
+        for (int hr = 0; hr < 6; ++hr)
+#pragma unroll
+            for (int kx = 0; kx < 3; ++kx) {
+                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(lds + ((r0 + hr) * HALO + j + kx) * PIX_BYTES + g * 16);
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) {
+                    const int ky = hr - rr;
+                    if (ky < 0 || ky > 2) continue;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) acc[rr][h] = mfma(wa[h][ky * 3 + kx], b, acc[rr][h]);
+                }
             }
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+            const int r = r0 + rr;
             const int gy = y0 + r, gx = x0 + j;
             if (gy >= H || gx >= W) continue;
             const long long pix = ((long long)n * H + gy) * W + gx;
-            if (mode == 1) {
-                if (g == 0) static_cast<float *>(y)[((long long)n * H + gy) * ostride + gx] = base[pix] + (acc[0] + bo[0]);
+            if (mode == 1) {  // the residual output layer: output channel 0
+                if (g == 0) static_cast<float *>(y)[((long long)n * H + gy) * ostride + gx] = base[pix] + (acc[rr][0][0] + bo[0]);
                 continue;
             }
-            float vv[4];
+            float vv[8];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) vv[q] = acc[q];
+            for (int q = 0; q < 8; ++q) vv[q] = acc[rr][q >> 2][q & 3];
             if (mode == 0) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) vv[q] = fmaxf(vv[q] + bo[q], 0.0f);
+                for (int q = 0; q < 8; ++q) vv[q] = fmaxf(vv[q] + bo[q], 0.0f);
             } else {
-                const uint2 m = *reinterpret_cast<const uint2 *>(aux + pix * CH + o);
-                const unsigned short mm[4] = {(unsigned short)(m.x & 0xffff), (unsigned short)(m.x >> 16),
-                                              (unsigned short)(m.y & 0xffff), (unsigned short)(m.y >> 16)};
+                const uint4 m = *reinterpret_cast<const uint4 *>(aux + pix * CH + o);
+                const unsigned mm[4] = {m.x, m.y, m.z, m.w};
 #pragma unroll
-                for (int q = 0; q < 4; ++q) vv[q] = bf2f(mm[q]) > 0.0f ? vv[q] : 0.0f;
+                for (int q = 0; q < 8; ++q) {
+                    const float av = __uint_as_float(q & 1 ? mm[q >> 1] & 0xffff0000u : mm[q >> 1] << 16);
+                    vv[q] = av > 0.0f ? vv[q] : 0.0f;
+                }
             }
-            bf16x4 o4;
+            bf16x8 o8;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) o4[q] = (__bf16)vv[q];
-            *reinterpret_cast<bf16x4 *>(static_cast<unsigned short *>(y) + pix * CH + o) = o4;
+            for (int q = 0; q < 8; ++q) o8[q] = (__bf16)vv[q];
+            *reinterpret_cast<bf16x8 *>(static_cast<unsigned short *>(y) + pix * CH + o) = o8;
         }
     }
 }
@@ -528,8 +545,8 @@ int vsz_cnn_conv3x3(const void *x, const void *w, const float *bias, int n, int 
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return vsz_fail(VSZ_EDEVICE, "vsz_cnn_conv3x3: no device");
-    // six workgroups per CU (their 26 KB halos fit the LDS together): measured best of 2..8
-    const int grid = (int)std::min<long long>(tiles, 6LL * std::max(cus, 1));
+    // as many as the registers let a CU hold
+    const int grid = (int)std::min<long long>(tiles, 2LL * std::max(cus, 1));
     hipLaunchKernelGGL(k_conv3x3, dim3(grid), dim3(256), 0, (hipStream_t)stream, (const unsigned short *)x,
                        (const unsigned short *)w, bias, n, h, wd, (int)tiles, mode, (const unsigned short *)aux, base, y,
                        out_stride);
