@@ -6,9 +6,10 @@ ps_num=2, ps_range=4, ssd, dct/dct, extractor_exp=3, float32. Inputs are synthet
 generator) and resident in HBM before the timed region. One step = both passes (matching,
 filtering, aggregation, division) over the frame. value = Mpix/s = 1920*1080 / step time.
 
-Roofline: the dominant kernel's algorithmic work is counted from the reference geometry:
-SSD_FLOP = 192 per candidate block evaluation, summed over the clipped windows of every
-reference block of both passes. Its duration comes from HIP events on the launch stream.
+Roofline: block matching, its duration from HIP events on the launch stream. `achieved` is the matrix work that the
+screened search executes (screen_flop); ssd_equivalent_tflops is the exhaustive search's algorithmic work, counted from the
+reference geometry, over the same time: SSD_FLOP = 192 per candidate block evaluation, summed over the
+clipped windows of every reference block of both passes.
 step_roofline: the whole step's lower bound T_min = (SSD_FLOP + TF_FLOP) / P_fp32, with
 TF_FLOP = 128 per 8-point transform (384 per group and plane for the hard pass, 576 for Wiener),
 against the measured step time.
@@ -58,6 +59,14 @@ CNN_FLOP_PER_PX = 2 * 9 * (2 * 32 + 4 * 32 * 32 + 32 * 1)
 
 def num_blocks(width, height, step):
     return len(origins(width, step)) * len(origins(height, step))
+
+
+def screen_flop(width, height, step, reach):
+    """Matrix work of one screened search: per 4 x 4 blocks two passes over the 3 step + 2 reach + 1 candidate rows and
+    columns, in groups of 4 rows by 16 columns of 11 products (16 x 16 x 32)."""
+    bx, by = len(origins(width, step)), len(origins(height, step))
+    span = 3 * step + 2 * reach + 1
+    return ((bx + 3) // 4) * ((by + 3) // 4) * 2 * ((span + 3) // 4) * ((span + 15) // 16) * 11 * 2 * 16 * 16 * 32
 
 
 def temporal_candidates(width, height, step, radius, ps_num, ps_range):
@@ -520,6 +529,7 @@ def main():
     cand = ssd_candidates(W, H, PARAMS["block_step"], PARAMS["bm_range"])
     flop = 192.0 * cand * 2
     achieved = flop / (t_match_b + t_match_f) / 1e12
+    screen = 2 * screen_flop(W, H, PARAMS["block_step"], PARAMS["bm_range"]) / (t_match_b + t_match_f) / 1e12
     t_match = t_match_b + t_match_f
     print(f"bench: match kernels {t_match_b * 1e3:.3f} + {t_match_f * 1e3:.3f} ms, "
           f"{cand} candidates/pass, {achieved:.2f} TFLOP/s", file=sys.stderr, flush=True)
@@ -648,12 +658,12 @@ def main():
                    "match_ms_per_step": round(t_match * 1e3, 4), "basic_pass_ms": round(t_basic * 1e3, 4),
                    "matcher": device.match_plan(kp_b),
                    "filter_tiles": {"basic": list(device.filter_plan(kp_b)), "wiener": list(device.filter_plan(kp_f))}},
-        "roofline": {"bound": "valu", "achieved": round(achieved, 3), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(achieved / PEAK_FP32_TFLOPS, 4), "traffic": traffic,
-                     "kernel": "k_match_lds4 (SSD block matching, both passes)",
-                     "work": "dense-equivalent SSD FLOP, 192 per candidate block; the kernel executes about half "
-                             "(each lane takes half of its distance tree from its neighbour) and issues VALU work "
-                             "on every SIMD cycle (profiles/k_match_lds4_1080p_valu_counters.md)"},
+        "roofline": {"bound": "mfma", "achieved": round(screen, 3), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
+                     "frac": round(screen / PEAK_BF16_TFLOPS, 4), "traffic": traffic,
+                     "ssd_equivalent_tflops": round(achieved, 3),
+                     "kernel": "k_match_screen + k_match_tied (SSD block matching, both passes)",
+                     "work": "half-precision products of the screened search; VALU issue beside them is what bounds it "
+                             "(profiles/k_match_screen_1080p_counters.md)"},
         "step_roofline": {"ssd_gflop": round(flop / 1e9, 3), "tf_gflop": round(tf_flop / 1e9, 3),
                           "t_min_ms": round(t_min * 1e3, 4), "frac": round(t_min / dt, 4)},
         "end_to_end_mpix_s": e2e,
