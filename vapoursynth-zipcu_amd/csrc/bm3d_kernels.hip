@@ -31,6 +31,7 @@
 
 #include "vszipcu_bm3d.h"
 #include "internal.h"
+#include "screen_geom.h"
 
 namespace vszk {
 
@@ -904,63 +905,6 @@ typedef float scr_f2 __attribute__((ext_vector_type(2)));
 typedef float scr_f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kScrMost = 384;  // candidates evaluated per wave (144 and up; on video with noise below 200)
-constexpr int kScrCap = 16;    // keys kept per block between two insertions
-constexpr int kScrLds8 = 20480;   // LDS bytes that each of 8 workgroups of a CU may take
-constexpr int kScrLdsMax = 40960;  // a quarter of the CU's
-
-struct ScreenGeom {
-    int ng, tiles;        // 4-row groups and 16-column tiles of a 4 x 4 block tile's candidates
-    int pw, ph, nc, nr;   // half-pixel region (pitch, rows); norm array (pitch, rows)
-    int queue;            // 8-byte results a wave can queue
-    int slack;            // zeroed halves past the region: reads of masked columns in its last row end there
-    int half_bytes, norm_bytes;
-    // how 64 lanes walk the region's pairs and the norms' segments: i / d = i * m >> 16 below 4096
-    int rstep, pair_m, segs, segs_m, vsegs, vsegs_m;
-};
-
-struct ScreenWave {  // per wave
-    unsigned long long kbuf[16 * kScrCap];  // (distance, position) keys to insert, per block
-    unsigned long long best[16 * 8];        // sorted keys of the best so far
-    unsigned cnt[16];
-    unsigned refpos[16];
-};
-
-// Bytes of the half region and of the norms (the last 8 rows of their first stage reach into the rest,
-// which is not in use yet).
-inline int screen_half_bytes(const ScreenGeom &G) { return ((G.pw * G.ph + G.slack) * 2 + 15) & ~15; }
-inline int screen_norm_bytes(const ScreenGeom &G) { return (G.nc * G.nr * 4 + 15) & ~15; }
-inline int screen_lds_bytes(const ScreenGeom &G) {
-    const int tail = 8 * G.nc * 4, rest = (int)sizeof(ScreenWave) + 8 * G.queue + 8;
-    return screen_half_bytes(G) + screen_norm_bytes(G) + (tail > rest ? tail : rest);
-}
-
-inline ScreenGeom screen_geom(int bs, int R, int nt) {
-    ScreenGeom G;
-    const int span = 3 * bs + 2 * R + 1;
-    G.ng = (span + 3) / 4;
-    G.tiles = ((span + 15) / 16 + nt - 1) / nt * nt;
-    G.pw = (span + 7 + 3) & ~3;   // columns past it belong to masked candidates only (they read on)
-    G.nc = (span + 1) & ~1;
-    if (G.nc % 16 == 0) G.nc += 2;   // rows of one column 12 apart in different banks
-    G.nr = 4 * G.ng;
-    G.ph = G.nr + 8;
-    G.slack = (16 * G.tiles + 64 - G.pw + 7) / 8 * 8;
-    G.slack = G.slack > 64 ? G.slack : 64;
-    G.half_bytes = screen_half_bytes(G);
-    G.norm_bytes = screen_norm_bytes(G);
-    const auto magic = [](int d) { return (65536 + d - 1) / d; };
-    G.rstep = G.pw / 2 <= 64 ? 64 / (G.pw / 2) : 1;
-    G.pair_m = magic(G.pw / 2 <= 64 ? G.pw / 2 : 64);
-    G.segs = (G.nc + 23) / 24;
-    G.segs_m = magic(G.segs);
-    G.vsegs = (G.nr + 11) / 12;
-    G.vsegs_m = magic(G.vsegs);
-    // the queue takes what is left of the LDS that lets 8 workgroups share a CU
-    G.queue = 256;
-    const int room = kScrLds8 - screen_lds_bytes(G);
-    G.queue += (room < 0 ? 0 : room > 8 * 64 ? 8 * 64 : room) / 8;
-    return G;
-}
 
 template <int CTRL> __device__ __forceinline__ int dpp_i(int v) {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
@@ -1133,18 +1077,19 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
     const bool inside = rx0 >= 0 && rx0 + G.pw <= W && ry0 >= 0 && ry0 + G.ph <= H;
     // d = (v - mid) * sc in one rounding (sc is a power of two); the largest |d|
     const auto convert = [&](float sc, bool bad) -> float {
-        constexpr int kRows = 28;
+        constexpr int kRows = kScrRows;
         const float off = -mid * sc;
         float big = 0.0f;
         for (int pr = spair; pr < p2; pr += 64) {
             const int gx = rx0 + 2 * pr;
             for (int r = srow; r < (srow < rstep ? G.ph : 0); r += kRows * rstep) {
                 float v[kRows][2];
-                if (inside) {   // rows past the region's end are inside the plane's buffer or read as 0
+                if (inside) {
                     const int at = ((ry0 + r) * S + gx) * 4, step = rstep * S * 4;
 #pragma unroll
                     for (int k = 0; k < kRows; ++k) {
-                        const vsz_u2 u = __builtin_bit_cast(vsz_u2, __builtin_amdgcn_raw_buffer_load_b64(img.rsrc, at, k * step, 0));
+                        const ScreenLoad ld = screen_region_load(at, k, step);
+                        const vsz_u2 u = __builtin_bit_cast(vsz_u2, __builtin_amdgcn_raw_buffer_load_b64(img.rsrc, ld.checked, ld.added, 0));
                         v[k][0] = __uint_as_float(u[0]);
                         v[k][1] = __uint_as_float(u[1]);
                     }
@@ -3176,14 +3121,6 @@ int tied_pitch(int bs, int R) { return (3 * bs + 2 * R + 12) | 1; }
 size_t tied_lds_bytes(int bs, int R) { return ((size_t)(2 * R + 8) * tied_pitch(bs, R) + 3) * 4; }
 int tied_wgs(int tiles) { return (int)std::min(4LL * tiles, 1024LL); }
 
-// Columns per product pass of the screened search: tiles of 16 in sets of two or three, whichever leaves
-// fewer.
-int screen_nt(int bs, int R) {
-    return screen_geom(bs, R, 2).tiles < screen_geom(bs, R, 3).tiles ? 2 : 3;
-}
-
-ScreenGeom screen_plan(int bs, int R) { return screen_geom(bs, R, screen_nt(bs, R)); }
-
 // Whether the screened search takes a spatial ssd search of so many 4 x 4 block tiles. Its cost per block hardly
 // depends on the window below 48 columns, the scan's grows with its area. Times of whole passes (scan / screened, us, frames
 // with noise and the same with letterbox bars, whose tiles are searched twice):
@@ -3193,8 +3130,6 @@ ScreenGeom screen_plan(int bs, int R) { return screen_geom(bs, R, screen_nt(bs, 
 // so it starts at 8 where one wave per SIMD takes all tiles and at 12 elsewhere; at 16 where its region exceeds an
 // eighth of a CU's LDS (block_step 8: 12 170/175 and 165/195, 16 229/184 and 224/231 at 1920x1080). Above a quarter
 // (bm_range 24 at block_step 8) it no longer gains.
-bool screen_fits(int bs, int R) { return R < 1024 && screen_lds_bytes(screen_plan(bs, R)) <= kScrLdsMax; }
-
 bool screen_pays(int bs, int R, long long tiles) {
     if (!screen_fits(bs, R)) return false;
     return R >= (tiles <= 512 ? 8 : screen_lds_bytes(screen_plan(bs, R)) <= kScrLds8 ? 12 : 16);

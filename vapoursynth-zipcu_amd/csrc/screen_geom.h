@@ -1,0 +1,90 @@
+// Geometry of the screened ssd search (k_match_screen, k_match_tied): region, norms and queue of one wave, their place in the
+// LDS, and the addresses of its loads. Host code plans with it, the kernels walk by it, and a CPU check
+// enumerates what they read.
+#pragma once
+
+namespace vszk {
+
+constexpr int kScrCap = 16;    // keys kept per block between two insertions
+constexpr int kScrLds8 = 20480;   // LDS bytes that each of 8 workgroups of a CU may take
+constexpr int kScrLdsMax = 40960;  // a quarter of the CU's
+constexpr int kScrRows = 28;   // region rows that a lane loads at a time, ScreenGeom::rstep apart
+
+struct ScreenGeom {
+    int ng, tiles;        // 4-row groups and 16-column tiles of a 4 x 4 block tile's candidates
+    int pw, ph, nc, nr;   // half-pixel region (pitch, rows); norm array (pitch, rows)
+    int queue;            // 8-byte results a wave can queue
+    int slack;            // zeroed halves past the region: reads of masked columns in its last row end there
+    int half_bytes, norm_bytes;
+    // how 64 lanes walk the region's pairs and the norms' segments: i / d = i * m >> 16 below 4096
+    int rstep, pair_m, segs, segs_m, vsegs, vsegs_m;
+};
+
+struct ScreenWave {  // per wave
+    unsigned long long kbuf[16 * kScrCap];  // (distance, position) keys to insert, per block
+    unsigned long long best[16 * 8];        // sorted keys of the best so far
+    unsigned cnt[16];
+    unsigned refpos[16];
+};
+
+// Bytes of the half region and of the norms (the last 8 rows of their first stage reach into the rest,
+// which is not in use yet).
+inline int screen_half_bytes(const ScreenGeom &G) { return ((G.pw * G.ph + G.slack) * 2 + 15) & ~15; }
+inline int screen_norm_bytes(const ScreenGeom &G) { return (G.nc * G.nr * 4 + 15) & ~15; }
+inline int screen_lds_bytes(const ScreenGeom &G) {
+    const int tail = 8 * G.nc * 4, rest = (int)sizeof(ScreenWave) + 8 * G.queue + 8;
+    return screen_half_bytes(G) + screen_norm_bytes(G) + (tail > rest ? tail : rest);
+}
+
+inline ScreenGeom screen_geom(int bs, int R, int nt) {
+    ScreenGeom G;
+    const int span = 3 * bs + 2 * R + 1;
+    G.ng = (span + 3) / 4;
+    G.tiles = ((span + 15) / 16 + nt - 1) / nt * nt;
+    G.pw = (span + 7 + 3) & ~3;   // columns past it belong to masked candidates only (they read on)
+    G.nc = (span + 1) & ~1;
+    if (G.nc % 16 == 0) G.nc += 2;   // rows of one column 12 apart in different banks
+    G.nr = 4 * G.ng;
+    G.ph = G.nr + 8;
+    G.slack = (16 * G.tiles + 64 - G.pw + 7) / 8 * 8;
+    G.slack = G.slack > 64 ? G.slack : 64;
+    G.half_bytes = screen_half_bytes(G);
+    G.norm_bytes = screen_norm_bytes(G);
+    const auto magic = [](int d) { return (65536 + d - 1) / d; };
+    G.rstep = G.pw / 2 <= 64 ? 64 / (G.pw / 2) : 1;
+    G.pair_m = magic(G.pw / 2 <= 64 ? G.pw / 2 : 64);
+    G.segs = (G.nc + 23) / 24;
+    G.segs_m = magic(G.segs);
+    G.vsegs = (G.nr + 11) / 12;
+    G.vsegs_m = magic(G.vsegs);
+    // the queue takes what is left of the LDS that lets 8 workgroups share a CU
+    G.queue = 256;
+    const int room = kScrLds8 - screen_lds_bytes(G);
+    G.queue += (room < 0 ? 0 : room > 8 * 64 ? 8 * 64 : room) / 8;
+    return G;
+}
+
+// A buffer load's byte offset: its range check covers `checked`; `added` (the scalar offset) is added past the
+// check.
+struct ScreenLoad {
+    int checked, added;
+};
+
+// Where a lane finds the pixels k steps of `step` bytes below those at `at`. Rows past the region may lie past the
+// plane, so all of it is checked: such loads return 0 and what they return is not used.
+constexpr ScreenLoad screen_region_load(int at, int k, int step) {
+    return ScreenLoad{(int)((unsigned)at + (unsigned)k * (unsigned)step), 0};
+}
+
+// Columns per product pass of the screened search: tiles of 16 in sets of two or three, whichever leaves
+// fewer.
+inline int screen_nt(int bs, int R) {
+    return screen_geom(bs, R, 2).tiles < screen_geom(bs, R, 3).tiles ? 2 : 3;
+}
+
+inline ScreenGeom screen_plan(int bs, int R) { return screen_geom(bs, R, screen_nt(bs, R)); }
+
+// Windows up to a quarter of a CU's LDS.
+inline bool screen_fits(int bs, int R) { return R < 1024 && screen_lds_bytes(screen_plan(bs, R)) <= kScrLdsMax; }
+
+}  // namespace vszk
