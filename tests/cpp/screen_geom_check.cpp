@@ -1,5 +1,6 @@
 // CPU check of the screened search's geometry (csrc/screen_geom.h), over every block step and window it takes: what
 // a wave reads of the plane, walked as k_match_screen walks it.
+#include <cstddef>
 #include <cstdio>
 
 #include "screen_geom.h"
@@ -30,12 +31,27 @@ static bool region_loads(int bs, int R, const ScreenGeom &G) {
     return true;
 }
 
+// The norms that rows of the search read: all of them before the keys kept behind the norms, and past the norms' rows
+// only what their first stage wrote (the sums of the 8 region rows below).
+static bool norm_reads(int bs, int R, const ScreenGeom &G) {
+    const int span = 3 * bs + 2 * R + 1;
+    for (int row = 0; row < span; ++row) {
+        const int last = row * G.nc + 16 * G.tiles - 1;
+        if (4 * (last + 1) > G.norm_bytes || last >= G.nc * (G.nr + 8)) {
+            std::printf("block_step %d bm_range %d: row %d reads norm %d of %d bytes\n", bs, R, row, last, G.norm_bytes);
+            return false;
+        }
+    }
+    // ... which ends before what the wave keeps there from its start
+    return G.norm_bytes + (int)offsetof(ScreenWave, cnt) >= 4 * G.nc * (G.nr + 8);
+}
+
 int main() {
     int n = 0;
     for (int bs = 1; bs <= 8; ++bs)
         for (int R = 1; screen_fits(bs, R); ++R, ++n) {
             const ScreenGeom G = screen_plan(bs, R);
-            if (!region_loads(bs, R, G)) return 1;
+            if (!region_loads(bs, R, G) || !norm_reads(bs, R, G)) return 1;
         }
     std::printf("screen geometry: ok, %d plans\n", n);
     return 0;

@@ -1,0 +1,35 @@
+"""The screened ssd search at the edges of what it accepts, against the FP32 oracle: match lists and distances bit for
+bit."""
+import numpy as np
+import pytest
+
+from gpu_util import assert_matches_equal, kp_and_op
+from vszipcu import device, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _match(torch, kp, img):
+    nbx, nby = device.num_blocks(kp)
+    m = torch.zeros((nby, nbx, 8, 4), dtype=torch.int32, device="cuda")
+    device.match(kp, img, m)
+    torch.cuda.synchronize()
+    return m.cpu().numpy()
+
+
+@pytest.mark.parametrize("bs,rng", [(5, 20), (3, 15)])
+def test_tall_plane(orc, torch_gpu, bs, rng):
+    """Rows beyond 32640, whose packed positions would be infinities and NaNs if they were read as floats; 4 rows divide
+    both windows, so the last searched row reads past the norms' pitch. The lower end of the plane is compared with the
+    oracle's search of that end alone."""
+    torch = torch_gpu
+    print(f"screened search: 64x32800 bs={bs} R={rng}", flush=True)
+    W, H, y0 = 64, 32800, 32400                     # 32400 is a multiple of both block steps
+    img = np.random.default_rng(bs).random((H, W), dtype=np.float32)
+    kp, _ = kp_and_op(orc, W, H, bs=bs, rng=rng)
+    _, op = kp_and_op(orc, W, H - y0, bs=bs, rng=rng)
+    om, oe = orc.match(op, np.ascontiguousarray(img[None, y0:]))
+    gm = _match(torch, kp, torch.from_numpy(img[None]).cuda())[y0 // bs:]
+    first = -(-rng // bs)                           # block rows whose windows stay inside the end
+    gm[..., 1] -= y0
+    assert_matches_equal(gm[first:], om[first:], oe[first:])

@@ -28,9 +28,14 @@ struct ScreenWave {  // per wave
 };
 
 // Bytes of the half region and of the norms (the last 8 rows of their first stage reach into the rest,
-// which is not in use yet).
+// which is not in use yet). Columns of the last tile past the norms' pitch belong to masked candidates and read
+// the next row; after the last row, which is searched where 4 rows divide the window, they read
+// values that the norms' two stages left there. What is kept behind must not be read as a norm: a mask cannot undo a NaN.
 inline int screen_half_bytes(const ScreenGeom &G) { return ((G.pw * G.ph + G.slack) * 2 + 15) & ~15; }
-inline int screen_norm_bytes(const ScreenGeom &G) { return (G.nc * G.nr * 4 + 15) & ~15; }
+inline int screen_norm_bytes(const ScreenGeom &G) {
+    const int over = 16 * G.tiles > G.nc ? 16 * G.tiles - G.nc : 0;
+    return ((G.nc * G.nr + over) * 4 + 15) & ~15;
+}
 inline int screen_lds_bytes(const ScreenGeom &G) {
     const int tail = 8 * G.nc * 4, rest = (int)sizeof(ScreenWave) + 8 * G.queue + 8;
     return screen_half_bytes(G) + screen_norm_bytes(G) + (tail > rest ? tail : rest);
