@@ -33,3 +33,18 @@ def test_tall_plane(orc, torch_gpu, bs, rng):
     first = -(-rng // bs)                           # block rows whose windows stay inside the end
     gm[..., 1] -= y0
     assert_matches_equal(gm[first:], om[first:], oe[first:])
+
+
+@pytest.mark.parametrize("stride", [(1 << 24) - 8, (1 << 24) + 8])
+def test_wide_stride(orc, torch_gpu, stride):
+    """Strides at both sides of 24 bits (a plane of 604 MB of which 64 columns are used)."""
+    torch = torch_gpu
+    print(f"screened search: 64x9 stride {stride}", flush=True)
+    W, H = 64, 9
+    img = np.random.default_rng(9).random((H, W), dtype=np.float32)
+    kp, _ = kp_and_op(orc, W, H, bs=1, rng=9, stride=stride)
+    _, op = kp_and_op(orc, W, H, bs=1, rng=9)
+    plane = torch.zeros((1, H, stride), device="cuda")
+    plane[0, :, :W] = torch.from_numpy(img).cuda()
+    om, oe = orc.match(op, img[None])
+    assert_matches_equal(_match(torch, kp, plane), om, oe)

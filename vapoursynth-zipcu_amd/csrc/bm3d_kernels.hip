@@ -3136,7 +3136,7 @@ bool screen_pays(int bs, int R, long long tiles) {
 }
 
 bool screened(const MatchArgs &a, int metric) {
-    return metric == 0 && screen_pays(a.block_step, a.bm_range, (long long)((a.nbx + 3) / 4) * ((a.nby + 3) / 4));
+    return metric == 0 && a.stride < kScrStrides && screen_pays(a.block_step, a.bm_range, (long long)((a.nbx + 3) / 4) * ((a.nby + 3) / 4));
 }
 
 struct MatchPlan {
@@ -4282,6 +4282,7 @@ int vsz_bm3d_batch_create(const vsz_bm3d_batch_params *bp, const vsz_bm3d_plane 
     }
     b->global_match = !b->lds_rows && !b->sc_allowed;  // windows beyond the LDS matchers' budget
     b->screen_ok = bp->metric == 0 && !b->global_match && screen_pays(bp->block_step, bp->bm_range, LLONG_MAX);
+    for (int i = 0; i < n; ++i) b->screen_ok = b->screen_ok && planes[i].stride < kScrStrides;
     b->use_matcher(b->sc_allowed);
     const float fac[2] = {bits_float(0x3f021bb6u), bits_float(0x3e40c0c1u)};  // src/bm3d.zig:1013-1024
     size_t acc = 0, rest = 0;

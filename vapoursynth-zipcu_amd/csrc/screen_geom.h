@@ -8,6 +8,7 @@ namespace vszk {
 constexpr int kScrCap = 16;    // keys kept per block between two insertions
 constexpr int kScrLds8 = 20480;   // LDS bytes that each of 8 workgroups of a CU may take
 constexpr int kScrLdsMax = 40960;  // a quarter of the CU's
+constexpr int kScrStrides = 1 << 24;   // strides below it: the exact evaluation multiplies rows by the stride in 24 bits
 constexpr int kScrRows = 28;   // region rows that a lane loads at a time, ScreenGeom::rstep apart
 
 struct ScreenGeom {
