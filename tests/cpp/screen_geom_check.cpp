@@ -50,7 +50,7 @@ int main() {
     int n = 0;
     for (int bs = 1; bs <= 8; ++bs)
         for (int R = 1; screen_fits(bs, R); ++R, ++n) {
-            const ScreenGeom G = screen_plan(bs, R);
+            const ScreenGeom G = screen_plan(bs, R, 1);
             if (!region_loads(bs, R, G) || !norm_reads(bs, R, G)) return 1;
         }
     std::printf("screen geometry: ok, %d plans\n", n);

@@ -884,10 +884,16 @@ __global__ __launch_bounds__(256) void k_match_lds4(MatchArgs a) {
 // Pass 1 finds a T' that 8 distinct candidates do not exceed; their exact distances, hence the 8
 // best, are below (sqrt((T' + 3c n_a)(1 + 3c)) + eps)^2, up to FP32 rounding; a candidate below that has
 // S' <= T'' (screen_limit). Pass 2 recomputes the products and passes on candidates with S' <= T''.
-// Queues are bounded: a full one is evaluated at once and the exact 8th distance tightens T''. A tile with
-// more than kScrMost candidates to evaluate, or with non-finite values, is marked and left to k_match_tied, which
-// searches it exhaustively: at about 130 cycles per gathered candidate, a wave that evaluated all of a tied
-// window took up to 570 k cycles (a usual one takes 50 to 97 k) and a small frame waited for it alone.
+// Queues are bounded: a full one is evaluated at once and the exact 8th distance tightens T''.
+//
+// Where more candidates pass than usual (ScreenGeom::most), the windows tie: areas of one value, drawn art, patterns.
+// A block that may have 8 zero distances then takes 8 candidates at a time in scan order, and once it has
+// them nothing later can enter; a block with more candidates than ScreenGeom::block that has not ended is left to
+// k_match_tied, and so are all blocks of a tile with values that are not finite. The marks are in the match list: the third
+// component of a block row's first entry, which no list uses, holds a bit per block. 1920x1080, block_step 4, bm_range 16, scan /
+// screened in us (before: a tile with more than 384 was left as a whole, before any was evaluated): flat drawn art 335 / 166 (711),
+// ordered dither 340 / 239 (1461), text 380 / 270 (496), art with noise of sigma 1 385 / 290 (419), noise with letterbox
+// bars 358 / 198 (285), noise 355 / 174 (172).
 //
 // What bounds it: VALU issue, about 30 instructions per candidate row of 16 blocks in pass 1 and 40 in
 // pass 2 with the products (11 per 4 rows and 16 columns, 16 cycles each) beside them, then the latency of
@@ -904,7 +910,7 @@ typedef _Float16 scr_h2 __attribute__((ext_vector_type(2)));
 typedef float scr_f2 __attribute__((ext_vector_type(2)));
 typedef float scr_f4 __attribute__((ext_vector_type(4)));
 
-constexpr int kScrMost = 384;  // candidates evaluated per wave (144 and up; on video with noise below 200)
+constexpr int kScrLane = 48;   // candidates that a lane queues before they are looked at: a 4-row group's
 
 template <int CTRL> __device__ __forceinline__ int dpp_i(int v) {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
@@ -936,10 +942,7 @@ __device__ __forceinline__ void key_insert(double (&L)[8], double k) {
     L[0] = key_min(L[0], k);
 }
 // The 8 smallest of two sorted lists, sorted.
-template <int CTRL> __device__ __forceinline__ void key_merge(double (&L)[8]) {
-    double b[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) b[i] = dpp_d<CTRL>(L[i]);
+__device__ __forceinline__ void key_merge(double (&L)[8], const double (&b)[8]) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) L[i] = key_min(L[i], b[7 - i]);
 #pragma unroll
@@ -951,6 +954,12 @@ template <int CTRL> __device__ __forceinline__ void key_merge(double (&L)[8]) {
                 L[i] = lo;
                 L[i + d] = hi;
             }
+}
+template <int CTRL> __device__ __forceinline__ void key_merge(double (&L)[8]) {
+    double b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) b[i] = dpp_d<CTRL>(L[i]);
+    key_merge(L, b);
 }
 
 // Floats as integers of the same order (its own inverse).
@@ -1137,8 +1146,8 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
     }
     lds_order();
 
-    bool tied = bad;   // left to k_match_tied
-    if (!flat && !tied) {
+    unsigned left = bad ? 0xffffu : 0u;   // blocks left to k_match_tied
+    if (!flat && !bad) {
         const float eps_floor = 1.0e-21f * sc;
 
         // -- norms: horizontal 8-sums of squares, then vertical ones in place ----------------------
@@ -1239,9 +1248,10 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
         };
         loadA();
         // squared norms of this lane's four result rows' blocks
-        float na[4];
+        const auto norms = [&](float (&na)[4]) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) na[q] = nh[(dyg + R) * G.nc + dxq[q] + R];
+            for (int q = 0; q < 4; ++q) na[q] = nh[(dyg + R) * G.nc + dxq[q] + R];
+        };
 
         const int chunks = G.tiles / NT;
         const int j0 = max(0, -ry0) >> 2;                                  // groups that meet the plane
@@ -1383,35 +1393,55 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
         }
         // The largest S' of a candidate whose exact distance has a root of at most re: its pixels differ
         // from the block's by no more than that, so they stay below |block| + re.
-        float rna[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) rna[q] = __builtin_amdgcn_sqrtf(na[q]) * 1.000001f;
-        const auto near_limit = [&](float re, int q) {
-            const float rt = re + screen_eps(fminf(big, (rna[q] + re) * 1.001f), eps_floor);
+        const auto root_norm = [](float n) { return __builtin_amdgcn_sqrtf(n) * 1.000001f; };
+        const auto near_limit = [&](float re, int q, const float (&na)[4]) {
+            const float rt = re + screen_eps(fminf(big, (root_norm(na[q]) + re) * 1.001f), eps_floor);
             return screen_limit(rt * rt * 1.00001f, na[q]);
         };
-        float th[4];
         {
-            float tau[4];
+            float tau[4], na[4];
+            unsigned zeros = 0u;   // bit q: 8 distances of block q may be 0
+            norms(na);
             eighth_of_64(m, lane, tau);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const float t1 = fmaxf(na[q] - 2.0f * tau[q], 0.0f);
+                zeros |= t1 <= 2.1f * kScrC * na[q] + 1.0e-5f ? 1u << q : 0u;
                 const float u1 = (t1 + 3.0f * kScrC * na[q]) * (1.0f + 3.0f * kScrC) + 1.0e-5f;
                 const float ru = __builtin_amdgcn_sqrtf(u1) * 1.000001f;
-                const float re = ru + screen_eps(fminf(big, (rna[q] + ru) * 1.001f), eps_floor);
-                th[q] = tau[q] > -inf ? 0.5f * (na[q] - near_limit(re, q)) : -3.0e38f;
+                const float re = ru + screen_eps(fminf(big, (root_norm(na[q]) + ru) * 1.001f), eps_floor);
+                if (n == 0) ws->th[g * 4 + q] = tau[q] > -inf ? 0.5f * (na[q] - near_limit(re, q, na)) : -3.0e38f;
             }
+            if (n == 0) ws->zeros[g] = zeros;
+            if (lane < 16) ws->seen[lane] = 0u;
+            lds_order();
         }
 
         // -- pass 2 ----------------------------------------------------------------------------------
+        // a result word of two rows: block 0's candidates (block q's are q bits lower) and the second row
+        constexpr unsigned kQ0 = NT == 3 ? 0x888888u : 0x8888u, kOdd = (1u << 4 * NT) - 1u;
         int ch = 0, j = j0, evaluated = 0;
         bool again = false;
-        while (ch < chunks && !tied) {
+        while (ch < chunks) {
             if (again) loadA();
             again = true;
             const int xs = 16 * NT * ch;
-            mask_cols(xs, th);
+            // nothing enters a list of 8 zero distances that comes after them in scan order
+            float now[4];
+            bool open = false;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const unsigned long long k = ws->best[(g * 4 + q) * 8 + 7];
+                const bool closed = ((unsigned)(k >> 32) == 0u && (int)((unsigned)k >> 16) < ry0 + 4 * j) || (left >> (g * 4 + q) & 1u);
+                now[q] = closed ? 3.0e38f : ws->th[g * 4 + q];
+                open |= !closed && bxm + q < a.nbx && bym + g < a.nby;
+            }
+            if (!__any(open)) {
+                ++ch;
+                j = j0;
+                continue;
+            }
+            mask_cols(xs, now);
             int queued = 0;
             int found = 0;   // this lane's candidates in the queue
             unsigned w[2];
@@ -1433,16 +1463,32 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
                     queue[(w0 | w1) != 0u ? at : (unsigned)G.queue] = vsz_u2{w0 | (unsigned)lane << 24, w1 | (unsigned)jj << 24};
                     queued += __builtin_popcountll(who);
                 }
-            }, [&] { return j < j1 && queued <= G.queue - 64 && !__any(found > 24); });
+            }, [&] { return j < j1 && queued <= G.queue - 64 && !__any(found > kScrLane); });
             if (j >= j1) {
                 ++ch;
                 j = j0;
             }
 
-            // too many even before the first of them is evaluated?
-            const int all = wave_sum(found);
-            tied = evaluated + all > kScrMost;
-            if (tied) break;
+            // many? Then blocks that will not end early and have too many are left
+            const bool many = evaluated + wave_sum(found) > G.most;
+            if (many && G.block == 0) {
+                left = 0xffffu;
+                break;
+            }
+            if (many) {
+                if (lane < 16) ws->cnt[lane] = 0u;
+                lds_order();
+                for (int i = lane; i < queued; i += 64) {
+                    const vsz_u2 e = queue[i];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        atomicAdd(&ws->cnt[(e[0] >> 28) * 4u + q], (unsigned)(__builtin_popcount(e[0] & kQ0 >> q) + __builtin_popcount(e[1] & kQ0 >> q)));
+                }
+                lds_order();
+                left |= (unsigned)__ballot(lane < 16 && !(ws->zeros[n >> 2] >> (n & 3) & 1u) && ws->cnt[n] + ws->seen[n] > (unsigned)G.block);
+                lds_order();
+                if (lane < 16) ws->cnt[lane] = 0u;
+            }
 
             // -- evaluate the queue, 8 lanes (columns) per candidate, 32 candidates at a time ----------
             lds_order();
@@ -1469,14 +1515,35 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
             const unsigned corner_pos = (unsigned)(ry0 * 65536 + rx0);
             int taken = 0;
             unsigned w0 = 0u, w1 = 0u, from = 0u, group = 0u;   // an entry's candidates that are not listed yet
+            // leaves out those of blocks that are left and those that come after their block's 8 zero distances
+            const auto drop = [&]() {
+                unsigned k0 = 0u, k1 = 0u;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const unsigned b = (from >> 4) * 4u + q;
+                    const unsigned long long k = ws->best[b * 8u + 7u];
+                    const int rows = (int)((unsigned)k >> 16) - ry0 - 4 * (int)group, x7 = (int)((unsigned)k & 0xffffu) - rx0 - xs - (int)(from & 15u);
+                    const bool all = (unsigned)(k >> 32) != 0u, none = left >> b & 1u;
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        const unsigned odd = 1u << (4 * NT - 1 - 4 * t - q), even = odd << 4 * NT;
+                        const int to = none ? 0 : all ? 4 : rows + (16 * t < x7 ? 1 : 0);   // rows of this group that stay
+                        k0 |= (to > 0 ? even : 0u) | (to > 1 ? odd : 0u);
+                        k1 |= (to > 2 ? even : 0u) | (to > 3 ? odd : 0u);
+                    }
+                }
+                w0 &= k0;
+                w1 &= k1;
+            };
             for (;;) {
                 // list candidates (block << 28 | row << 14 | column) in the space of the entries taken
                 int listed = 0;
+                unsigned full = 0u;   // candidates of blocks whose 8 are listed
                 for (;;) {
-                    const unsigned long long who = __ballot((w0 | w1) != 0u);
-                    const int more = __builtin_popcountll(who);
+                    const unsigned a0 = w0 & ~full, a1 = w1 & ~full;
+                    const int more = __builtin_popcountll(__ballot((a0 | a1) != 0u));
                     if (more == 0) {
-                        if (taken >= queued) break;
+                        if (taken >= queued || (many && __any((w0 | w1) != 0u))) break;
                         const vsz_u2 e = taken + lane < queued ? queue[taken + lane] : vsz_u2{0u, 0u};
                         lds_order();
                         w0 = e[0] & 0xffffffu;
@@ -1484,22 +1551,37 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
                         from = e[0] >> 24;
                         group = e[1] >> 24;
                         taken += 64;
+                        if (many) drop();
                         continue;
                     }
                     if (listed + more > 2 * (taken < queued ? taken : G.queue)) break;
-                    if ((w0 | w1) != 0u) {
-                        const bool second = w0 == 0u;
-                        const unsigned w = second ? w1 : w0;
-                        const int top = __builtin_clz(w), o = top - (32 - 8 * NT);      // order of evaluation
-                        const unsigned rest = w & ~(0x80000000u >> top);
-                        w1 = second ? rest : w1;
-                        w0 = second ? 0u : rest;
-                        const int odd = o >= 4 * NT ? 1 : 0, tq = o - odd * 4 * NT;
+                    const bool second = a0 == 0u;
+                    const unsigned w = second ? a1 : a0;
+                    bool take = w != 0u;
+                    const int top = take ? __builtin_clz(w) : 31, o = top - (32 - 8 * NT);      // order of evaluation
+                    const int odd = o >= 4 * NT ? 1 : 0, tq = o - odd * 4 * NT;
+                    const unsigned block = (from >> 4) * 4u + (unsigned)(tq & 3);
+                    if (many && take) {
+                        take = atomicAdd(&ws->cnt[block], 1u) < 8u || !(ws->zeros[block >> 2] >> (block & 3u) & 1u);
+                        full |= take ? 0u : kQ0 >> (tq & 3);
+                    }
+                    const unsigned long long who = __ballot(take);
+                    if (take) {
+                        const unsigned rest = ~(0x80000000u >> top);
+                        w1 &= second ? rest : ~0u;
+                        w0 &= second ? ~0u : rest;
                         list[__builtin_amdgcn_mbcnt_hi((unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, (unsigned)listed))] =
-                            ((from >> 4) * 4u + (unsigned)(tq & 3)) << 28 | (4u * group + (second ? 2u : 0u) + (unsigned)odd) << 14 |
+                            block << 28 | (4u * group + (second ? 2u : 0u) + (unsigned)odd) << 14 |
                             ((unsigned)(xs + 16 * (tq >> 2)) + (from & 15u));
                     }
-                    listed += more;
+                    listed += __builtin_popcountll(who);
+                }
+                if (many) {
+                    lds_order();
+                    if (lane < 16) {
+                        ws->seen[lane] += ws->zeros[lane >> 2] >> (lane & 3) & 1u ? min(ws->cnt[lane], 8u) : ws->cnt[lane];
+                        ws->cnt[lane] = 0u;
+                    }
                 }
                 if (listed == 0) break;
                 lds_order();
@@ -1571,17 +1653,22 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
                     fetch(f + 64, b0);
                     if (f + 32 < listed) evaluate(f + 32, b1);
                 }
+                evaluated += listed;
+                if (many) {
+                    insert();
+                    left |= (unsigned)__ballot(lane < 16 && ws->seen[n] > (unsigned)G.block && (ws->best[n * 8 + 7] >> 32) != 0ull);
+                    drop();
+                }
             }
             insert();
-            evaluated += all;
+            float na[4];
+            norms(na);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                // with one chunk what follows are later rows: none enters a list of 8 zero distances
                 const float e7 = __uint_as_float((unsigned)(ws->best[(g * 4 + q) * 8 + 7] >> 32));
-                if (e7 == 0.0f && chunks == 1) th[q] = 3.0e38f;
-                else if (e7 < FLT_MAX) {
-                    const float lim = near_limit(__builtin_sqrtf(e7) * sc * 1.000002f, q);
-                    if (lim < FLT_MAX) th[q] = max_nan(th[q], 0.5f * (na[q] - lim));
+                if (e7 < FLT_MAX) {
+                    const float lim = near_limit(__builtin_sqrtf(e7) * sc * 1.000002f, q, na);
+                    if (lim < FLT_MAX && n == 0) ws->th[g * 4 + q] = max_nan(ws->th[g * 4 + q], 0.5f * (na[q] - lim));
                 }
             }
             lds_order();
@@ -1599,10 +1686,6 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
             ws->best[i] = row < ny ? (unsigned long long)pack_xy(xa + k - row * nx, ya + row)
                                    : (unsigned long long)__float_as_uint(FLT_MAX) << 32;
         }
-    }
-    if (tied) {   // a third component of 1, which no list has, marks each block row of the tile
-        if (lane < 4 && bym + lane < a.nby) a.matches[((long long)(bym + lane) * a.nbx + bxm) * 8] = make_int4(0, 0, 1, 0);
-        return;
     }
     lds_order();
 
@@ -1626,8 +1709,10 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
         const int bx = bxm + (rf & 3), by = bym + (rf >> 2);
         const unsigned long long key = ws->best[i];
         const unsigned pos = (unsigned)key;
+        // the third component of a block row's first entry, 0 in a list, names the row's blocks that are left
         if (bx < a.nbx && by < a.nby)
-            a.matches[((long long)by * a.nbx + bx) * 8 + (i & 7)] = make_int4(pos_x(pos), pos_y(pos), 0, (int)(key >> 32));
+            a.matches[((long long)by * a.nbx + bx) * 8 + (i & 7)] =
+                make_int4(pos_x(pos), pos_y(pos), (i & 31) == 0 ? (int)(left >> (rf & 12) & 15u) : 0, (int)(key >> 32));
     }
 }
 
@@ -1638,26 +1723,40 @@ __global__ __launch_bounds__(64, 2) void k_match_screen(MatchArgs a, ScreenGeom 
     zero_share(a);
 }
 
-// The tiles that the screen left: areas so even (letterbox bars after a first pass, graphics) that whole windows are
-// within its bounds, and tiles with non-finite values. Such tiles are few and the search waits for the longest, so
-// each is four workgroups, one per block row, and a wave searches one block: its lanes take half a search row
-// each in turn, from the region staged in LDS, and their lists merge as keys. VALU issue bounds a lane's
-// candidates, about 1100 cycles each. With one workgroup per tile and 16 lanes per block, a 128x96 frame with bars
-// took 131 us at block_step 4, bm_range 16, and 96 so (the scan alone: 178).
-__device__ __forceinline__ void match_tied_body(const MatchArgs &a, int LS, int tile, int row, float *region) {
-    const int lane = threadIdx.x & 63;
+// The blocks that the screen left. They may be few, and the search then waits for the longest: a workgroup takes a block row of
+// four, and where one or two of them are left, its four waves share each. The lanes take parts of search rows from
+// the region staged in LDS in scan order, and their lists merge as keys. VALU issue bounds a lane's candidates, about
+// 1100 cycles each. With half rows of two for 64 lanes, in two rounds of which the second was nearly empty at bm_range 16, and
+// keys inserted one by one, a 128x96 frame with bars took 71 us at block_step 4, bm_range 16 with the search before it, and 54 so (the
+// scan: 154).
+__device__ __forceinline__ void match_tied_body(const MatchArgs &a, int LS, int segs1, int segs4, int tile, int row, unsigned blocks, float *region,
+                                               double (*lists)[8]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int W = a.width, H = a.height, S = a.stride, bs = a.block_step, R = a.bm_range;
-    const int bxm = tile % a.tiles_x * 4, by = tile / a.tiles_x * 4 + row, bx = bxm + (int)(threadIdx.x >> 6);
-    const int y = min(min(by, a.nby - 1) * bs, H - 8), x = min(min(bx, a.nbx - 1) * bs, W - 8);
+    const int bxm = tile % a.tiles_x * 4, by = tile / a.tiles_x * 4 + row;
+    const int y = min(by * bs, H - 8);
     const int rx0 = min(bxm * bs, W - 8) - R, ry0 = y - R, RH = 2 * R + 8;
     const int RW = min(min(bxm + 3, a.nbx - 1) * bs, W - 8) + R + 9 - rx0;   // (the scan loads a column ahead)
-    for (int Y = threadIdx.x >> 6; Y < RH; Y += 4)
-        for (int X = lane; X < RW; X += 64) {
-            const int gy = ry0 + Y, gx = rx0 + X;
-            region[lds_row(Y, LS) + X] = gy >= 0 && gy < H && gx >= 0 && gx < W ? a.img[(long long)gy * S + gx] : 0.0f;
+    for (int X = lane; X < RW; X += 64)
+        for (int Y0 = wave; Y0 < RH; Y0 += 4 * 10) {
+            const int gx = rx0 + X;
+            float v[10];
+#pragma unroll
+            for (int k = 0; k < 10; ++k) {
+                const int gy = ry0 + Y0 + 4 * k;
+                v[k] = Y0 + 4 * k < RH && gy >= 0 && gy < H && gx >= 0 && gx < W ? a.img[(long long)gy * S + gx] : 0.0f;
+            }
+#pragma unroll
+            for (int k = 0; k < 10; ++k)
+                if (Y0 + 4 * k < RH) region[lds_row(Y0 + 4 * k, LS) + X] = v[k];
         }
     __syncthreads();
-    if (bx < a.nbx && by < a.nby) {
+    // one or two blocks: the four waves share each; more: a wave takes one
+    const bool share = __builtin_popcount(blocks) <= 2;
+    const int segs = share ? segs4 : segs1, lanes = share ? 256 : 64, id = share ? (int)threadIdx.x : lane;
+    const int cols = (2 * R + segs) / segs;   // of a lane's part of a row
+    for (unsigned todo = share ? blocks : blocks & 1u << wave; todo; todo &= todo - 1) {
+        const int bx = bxm + __builtin_ctz(todo), x = min(bx * bs, W - 8);
         RefPatch ref;
 #pragma unroll
         for (int r = 0; r < 8; ++r)
@@ -1665,9 +1764,15 @@ __device__ __forceinline__ void match_tied_body(const MatchArgs &a, int LS, int 
             for (int c = 0; c < 8; ++c) ref.a[r * 8 + c] = region[lds_row(R + r, LS) + x + c - rx0];
         List8 L;
         list_init<false>(L, 0);
-        for (int h = lane; h < 2 * (2 * R + 1); h += 64) {   // columns -R..-1 and 0..R of each row
-            const int dy = (h >> 1) - R, x0 = h & 1 ? x : x - R;
-            lds_scan<0>(region, LS, x0 - rx0, ry0, W, H, x0, y, h & 1 ? R : R - 1, dy, dy + 1, ref, L);
+        for (int h = id; h < segs * (2 * R + 1); h += lanes) {
+            const int dy = h / segs - R, c0 = h % segs * cols, span = min(cols, 2 * R + 1 - c0) - 1;
+            lds_scan<0>(region, LS, x - R + c0 - rx0, ry0, W, H, x - R + c0, y, span, dy, span < 0 ? dy : dy + 1, ref, L);
+            if (!share) {   // parts are taken in scan order: after 8 zero distances nothing enters
+                int z = 0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) z += __builtin_popcountll(__ballot(L.er[k] == 0.0f));
+                if (z >= 8) break;
+            }
         }
         double K[8];
 #pragma unroll
@@ -1680,63 +1785,83 @@ __device__ __forceinline__ void match_tied_body(const MatchArgs &a, int LS, int 
             double o[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) o[k] = __shfl_xor(K[k], d);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) key_insert(K, o[k]);
+            key_merge(K, o);
         }
-        unsigned long long out[8];
-        const unsigned self = pack_xy(x, y);
-        bool found = a.no_self != 0;
+        if (share) {
+            if (lane == 0)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            out[k] = __builtin_bit_cast(unsigned long long, K[k]);
-            found |= (unsigned)out[k] == self;
-        }
-        if (!found) {
+                for (int k = 0; k < 8; ++k) lists[wave][k] = K[k];
+            __syncthreads();
+            if (wave == 0)
+                for (int w = 1; w < 4; ++w) {
+                    double o[8];
 #pragma unroll
-            for (int k = 7; k > 0; --k) out[k] = out[k - 1];
-            out[0] = self;
+                    for (int k = 0; k < 8; ++k) o[k] = lists[w][k];
+                    key_merge(K, o);
+                }
         }
-        if (lane == 0) {
+        if (lane == 0 && (wave == 0 || !share)) {
+            unsigned long long out[8];
+            const unsigned self = pack_xy(x, y);
+            bool found = a.no_self != 0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                out[k] = __builtin_bit_cast(unsigned long long, K[k]);
+                found |= (unsigned)out[k] == self;
+            }
+            if (!found) {
+#pragma unroll
+                for (int k = 7; k > 0; --k) out[k] = out[k - 1];
+                out[0] = self;
+            }
             int4 *o = a.matches + ((long long)by * a.nbx + bx) * 8;
 #pragma unroll
             for (int k = 0; k < 8; ++k) o[k] = make_int4(pos_x((unsigned)out[k]), pos_y((unsigned)out[k]), 0, (int)(out[k] >> 32));
         }
+        if (share) __syncthreads();   // the lists before the next block's
     }
-    __syncthreads();   // the region before the next tile's
+    __syncthreads();   // the region before the next row's
 }
 
-// Runs match_tied_body on the marked block rows of `tiles` tiles; plane(t, tile) gives a tile's arguments and its number
-// there.
+// Runs match_tied_body on the block rows of `tiles` tiles that have blocks left; plane(t, tile) gives a tile's arguments and its
+// number there.
 template <class Plane>
-__device__ __forceinline__ void match_tied(int tiles, int LS, float *region, const Plane &plane) {
-    __shared__ unsigned long long marked[4];
+__device__ __forceinline__ void match_tied(int tiles, int LS, int segs1, int segs4, float *region, const Plane &plane) {
+    __shared__ unsigned left[256];
+    __shared__ unsigned long long any[4];
+    __shared__ double lists[4][8];
     const int per = gridDim.x;
     for (int u0 = blockIdx.x; u0 < 4 * tiles; u0 += 256 * per) {
         const int u = u0 + (int)threadIdx.x * per;   // neighbours go to different workgroups
-        bool on = false;
+        unsigned m = 0u;
         if (u < 4 * tiles) {
             int tile;
             const MatchArgs &a = plane(u >> 2, tile);
-            const int by = tile / a.tiles_x * 4 + (u & 3);
-            on = by < a.nby && a.matches[((long long)by * a.nbx + tile % a.tiles_x * 4) * 8].z == 1;
+            const int by = tile / a.tiles_x * 4 + (u & 3), bx = tile % a.tiles_x * 4;
+            if (by < a.nby) {
+                int4 *first = a.matches + ((long long)by * a.nbx + bx) * 8;
+                m = (unsigned)first->z & (1u << min(4, a.nbx - bx)) - 1u;
+                if (m && !(m & 1u)) first->z = 0;   // the first block has its list: its mark goes
+            }
         }
-        const unsigned long long who = __ballot(on);
-        if ((threadIdx.x & 63) == 0) marked[threadIdx.x >> 6] = who;
+        left[threadIdx.x] = m;
+        const unsigned long long who = __ballot(m != 0u);
+        if ((threadIdx.x & 63) == 0) any[threadIdx.x >> 6] = who;
         __syncthreads();
         for (int w = 0; w < 4; ++w)
-            for (unsigned long long m = marked[w]; m; m &= m - 1) {
-                const int v = u0 + (64 * w + __builtin_ctzll(m)) * per;
+            for (unsigned long long b = any[w]; b; b &= b - 1) {
+                const int i = 64 * w + __builtin_ctzll(b), v = u0 + i * per;
                 int tile;
                 const MatchArgs &a = plane(v >> 2, tile);
-                match_tied_body(a, LS, tile, v & 3, region);
+                match_tied_body(a, LS, segs1, segs4, tile, v & 3, left[i], region, lists);
             }
         __syncthreads();
     }
 }
 
-__global__ __launch_bounds__(256) void k_match_tied(MatchArgs a, int tiles, int LS) {
+__global__ __launch_bounds__(256) void k_match_tied(MatchArgs a, int tiles, int LS, int segs1, int segs4) {
     extern __shared__ __align__(16) float region[];
-    match_tied(tiles, LS, region, [&](int t, int &tile) -> const MatchArgs & {
+    match_tied(tiles, LS, segs1, segs4, region, [&](int t, int &tile) -> const MatchArgs & {
         tile = t;
         return a;
     });
@@ -2849,9 +2974,9 @@ __global__ __launch_bounds__(64, 2) void k_match_screen_batch(const BatchTable *
     zero_range(zero, zero_n64);
 }
 
-__global__ __launch_bounds__(256) void k_match_tied_batch(const BatchTable *__restrict__ tab, int tiles, int LS) {
+__global__ __launch_bounds__(256) void k_match_tied_batch(const BatchTable *__restrict__ tab, int tiles, int LS, int segs1, int segs4) {
     extern __shared__ __align__(16) float region[];
-    match_tied(tiles, LS, region, [&](int t, int &tile) -> const MatchArgs & {
+    match_tied(tiles, LS, segs1, segs4, region, [&](int t, int &tile) -> const MatchArgs & {
         const int p = batch_plane(tab->match_off, tab->n, t);
         tile = t - tab->match_off[p];
         return tab->m[p];
@@ -3119,24 +3244,44 @@ enum MatchKernel { kMkLds4 = 0, kMkLds1, kMkLds2, kMkLds4Bands, kMkLdsShort, kMk
 // 30 KB where the screen runs; workgroups, which share out the marked block rows.
 int tied_pitch(int bs, int R) { return (3 * bs + 2 * R + 12) | 1; }
 size_t tied_lds_bytes(int bs, int R) { return ((size_t)(2 * R + 8) * tied_pitch(bs, R) + 3) * 4; }
+// ... and the parts that its 256 lanes cut a search row into: fewest steps, with one for a part's first columns
+int tied_segs(int R, int lanes, bool fine) {
+    int best = 1, least = INT_MAX;
+    for (int s = 1; s <= 2 * R + 1; ++s) {
+        const int steps = (s * (2 * R + 1) + lanes - 1) / lanes * ((2 * R + s) / s + 1);
+        if (steps < least || (fine && steps * 8 <= least * 9)) best = s;   // finer parts end earlier where distances are 0
+        least = std::min(least, steps);
+    }
+    return best;
+}
 int tied_wgs(int tiles) { return (int)std::min(4LL * tiles, 1024LL); }
 
-// Whether the screened search takes a spatial ssd search of so many 4 x 4 block tiles. Its cost per block hardly
-// depends on the window below 48 columns, the scan's grows with its area. Times of whole passes (scan / screened, us, frames
-// with noise and the same with letterbox bars, whose tiles are searched twice):
-//   tiles   240: bm_range 8 71/59 and 71/70, 9 77/60 and 76/70, 16 157/81 and 158/109 (640x360, block_step 8)
-//   tiles   920: bm_range 8 97/94 and 97/105, 9 106/97 and 104/107, 12 136/115 and 135/131, 16 179/113 and 179/146
-//   tiles  8160: bm_range 9 251/227 and 244/251, 12 336/263 and 330/302, 16 477/278 and 473/361 (1920x1080, block_step 4)
-// so it starts at 8 where one wave per SIMD takes all tiles and at 12 elsewhere; at 16 where its region exceeds an
-// eighth of a CU's LDS (block_step 8: 12 170/175 and 165/195, 16 229/184 and 224/231 at 1920x1080). Above a quarter
-// (bm_range 24 at block_step 8) it no longer gains.
-bool screen_pays(int bs, int R, long long tiles) {
+// Whether the screened search takes a spatial ssd search of so many 4 x 4 block tiles; `shared` where the
+// shared-column scan would. Its cost per tile follows the products (window and block steps rounded up to 16 columns), the scan's
+// the candidates, and the screen's is higher where windows tie, by what k_match_tied searches again. The rule takes what gains on
+// noise and costs little on the hardest of six contents (bars, drawn art without and with noise of sigma 1, text,
+// ordered dither, a radial gradient in 8 bits). Search time / scan time, on noise and on the hardest:
+//   up to 256 tiles (a wave per CU)   8/9 at 640x360 (240 tiles): 0.76 and 1.11; 8/12: 0.64 and 0.87; 2/9 at 128x96: 0.71 and 1.14
+//                                     (not 8/8 at 640x360: 0.84 and 1.20)
+//   up to 512   8/12 at 960x540: 0.66 and 1.10; 6/12 at 640x360: 0.50 and 0.86 (not 8/9: 0.80 and 1.40, 6/9: 0.80 and 1.33)
+//   above       4/12 at 640x360: 0.50 and 0.93; 6/12 at 1920x1080: 0.54 and 0.90; 2/12: 0.41 and 0.57; 4/16: 0.49 and 0.71, at
+//               3840x2160 0.55 and 1.28 (not 4/9 at 640x360: 0.65 and 1.33, 3/9: 0.76 and 1.51)
+//   the shared-column scan is twice as fast above 2048 tiles   (not 4/12 at 1280x720: 0.78 and 1.26, 2560x1440: 0.80 and 1.38,
+//               3840x2160: 0.83 and 1.76)
+//   beyond an eighth of a CU's LDS   8/16 at 1280x720 (920 tiles): 0.55 and 1.11; 6/16 at 1920x1080: 0.55 and 0.84; 4/20: 0.58 and
+//               0.75; with fewer candidates in its products and more than 1024 tiles it loses (8/16 at 1920x1080: 0.77 and 1.65)
+// (block_step/bm_range).
+bool screen_pays(int bs, int R, long long tiles, bool shared) {
     if (!screen_fits(bs, R)) return false;
-    return R >= (tiles <= 512 ? 8 : screen_lds_bytes(screen_plan(bs, R)) <= kScrLds8 ? 12 : 16);
+    if (tiles <= 512) return R >= (tiles <= 256 ? 9 : 12);
+    const ScreenGeom G = screen_plan(bs, R, tiles);
+    if (screen_lds_bytes(G) > kScrLds8) return R >= 16 && (tiles <= 1024 || screen_share(G, R) >= 0.29f);
+    return R >= (shared && tiles > 2048 ? 16 : 12);
 }
 
 bool screened(const MatchArgs &a, int metric) {
-    return metric == 0 && a.stride < kScrStrides && screen_pays(a.block_step, a.bm_range, (long long)((a.nbx + 3) / 4) * ((a.nby + 3) / 4));
+    return metric == 0 && a.stride < kScrStrides &&
+           screen_pays(a.block_step, a.bm_range, (long long)((a.nbx + 3) / 4) * ((a.nby + 3) / 4), a.block_step == 4 && (a.width - 8) % 4 == 0);
 }
 
 struct MatchPlan {
@@ -3178,14 +3323,14 @@ MatchPlan plan_match(const MatchArgs &a, int metric) {
 template <int M> void launch_spatial(const MatchArgs &a, const MatchPlan &pl, hipStream_t s) {
     MatchArgs b = a;
     if (screened(a, M)) {
-        const ScreenGeom G = screen_plan(a.block_step, a.bm_range);
-        const size_t lds = screen_lds_bytes(G);
         b.tiles_x = (a.nbx + 3) / 4;
         const dim3 grid((unsigned)(b.tiles_x * ((a.nby + 3) / 4)));
+        const ScreenGeom G = screen_plan(a.block_step, a.bm_range, (long long)grid.x);
+        const size_t lds = screen_lds_bytes(G);
         if (screen_nt(a.block_step, a.bm_range) == 2) hipLaunchKernelGGL(k_match_screen<2>, grid, dim3(64), lds, s, b, G);
         else hipLaunchKernelGGL(k_match_screen<3>, grid, dim3(64), lds, s, b, G);
         hipLaunchKernelGGL(k_match_tied, dim3(tied_wgs((int)grid.x)), dim3(256), tied_lds_bytes(a.block_step, a.bm_range), s, b,
-                           (int)grid.x, tied_pitch(a.block_step, a.bm_range));
+                           (int)grid.x, tied_pitch(a.block_step, a.bm_range), tied_segs(a.bm_range, 64, G.block == 0), tied_segs(a.bm_range, 256, false));
         return;
     }
     b.lds_stride = pl.lds_stride;
@@ -3756,11 +3901,12 @@ void launch_match_batch(int metric, bool shared_cols, const BatchTable *d, int w
 
 void launch_match_screen_batch(int bs, int R, const BatchTable *d, int wgs, unsigned long long *zero, long long n64,
                                hipStream_t s) {
-    const ScreenGeom G = screen_plan(bs, R);
+    const ScreenGeom G = screen_plan(bs, R, wgs);
     const size_t lds = screen_lds_bytes(G);
     if (screen_nt(bs, R) == 2) hipLaunchKernelGGL(k_match_screen_batch<2>, dim3(wgs), dim3(64), lds, s, d, G, zero, n64);
     else hipLaunchKernelGGL(k_match_screen_batch<3>, dim3(wgs), dim3(64), lds, s, d, G, zero, n64);
-    hipLaunchKernelGGL(k_match_tied_batch, dim3(tied_wgs(wgs)), dim3(256), tied_lds_bytes(bs, R), s, d, wgs, tied_pitch(bs, R));
+    hipLaunchKernelGGL(k_match_tied_batch, dim3(tied_wgs(wgs)), dim3(256), tied_lds_bytes(bs, R), s, d, wgs, tied_pitch(bs, R),
+                       tied_segs(R, 64, G.block == 0), tied_segs(R, 256, false));
 }
 
 void launch_match_global_batch(int metric, const BatchTable *d, int wgs, unsigned long long *zero, long long n64,
@@ -4281,7 +4427,7 @@ int vsz_bm3d_batch_create(const vsz_bm3d_batch_params *bp, const vsz_bm3d_plane 
         b->sc_allowed = b->lds_sc != 0;
     }
     b->global_match = !b->lds_rows && !b->sc_allowed;  // windows beyond the LDS matchers' budget
-    b->screen_ok = bp->metric == 0 && !b->global_match && screen_pays(bp->block_step, bp->bm_range, LLONG_MAX);
+    b->screen_ok = bp->metric == 0 && !b->global_match && screen_pays(bp->block_step, bp->bm_range, LLONG_MAX, b->sc_allowed);
     for (int i = 0; i < n; ++i) b->screen_ok = b->screen_ok && planes[i].stride < kScrStrides;
     b->use_matcher(b->sc_allowed);
     const float fac[2] = {bits_float(0x3f021bb6u), bits_float(0x3e40c0c1u)};  // src/bm3d.zig:1013-1024

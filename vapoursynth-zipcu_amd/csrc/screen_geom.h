@@ -17,6 +17,9 @@ struct ScreenGeom {
     int queue;            // 8-byte results a wave can queue
     int slack;            // zeroed halves past the region: reads of masked columns in its last row end there
     int half_bytes, norm_bytes;
+    // candidates that a wave evaluates as they come (usually 144 and up, below 200 on video with noise); where there are more, those
+    // it evaluates for a block before it leaves the block (0: it leaves the tile at once)
+    int most, block;
     // how 64 lanes walk the region's pairs and the norms' segments: i / d = i * m >> 16 below 4096
     int rstep, pair_m, segs, segs_m, vsegs, vsegs_m;
 };
@@ -26,6 +29,9 @@ struct ScreenWave {  // per wave
     unsigned long long best[16 * 8];        // sorted keys of the best so far
     unsigned cnt[16];
     unsigned refpos[16];
+    float th[16];                           // least result that passes in the second pass
+    unsigned seen[16];                      // candidates evaluated while there were many
+    unsigned zeros[4];                      // per block row, bit q: block q may have 8 distances of 0
 };
 
 // Bytes of the half region and of the norms (the last 8 rows of their first stage reach into the rest,
@@ -88,9 +94,24 @@ inline int screen_nt(int bs, int R) {
     return screen_geom(bs, R, 2).tiles < screen_geom(bs, R, 3).tiles ? 2 : 3;
 }
 
-inline ScreenGeom screen_plan(int bs, int R) { return screen_geom(bs, R, screen_nt(bs, R)); }
+// Which blocks a wave leaves to k_match_tied depends on what the search waits for. Up to 512 tiles leave most of the chip
+// idle, so leaving a tile is quickest (640x360, block_step 8, bm_range 9, flat drawn art: 49 us, 77 with 24 and 90 with 96 for a
+// block); up to 2048, all waves at once, the last wave counts (960x540, block_step 4, bm_range 12, art with noise: 384 and 24 take 94 us,
+// 384 and 96 108); above, the work does (1920x1080, block_step 4, bm_range 12, text: 384 and 24 260 us, 1000 and 96 226; ordered
+// dither at bm_range 16: 1080 and 248).
+inline ScreenGeom screen_plan(int bs, int R, long long tiles) {
+    ScreenGeom G = screen_geom(bs, R, screen_nt(bs, R));
+    G.most = tiles <= 2048 ? 384 : 1000;
+    G.block = tiles <= 512 ? 0 : tiles <= 2048 ? 24 : 96;
+    return G;
+}
+
+// Candidates among the products' results.
+inline float screen_share(const ScreenGeom &G, int R) {
+    return (float)((2 * R + 1) * (2 * R + 1)) / (float)(4 * G.ng * 16 * G.tiles);
+}
 
 // Windows up to a quarter of a CU's LDS.
-inline bool screen_fits(int bs, int R) { return R < 1024 && screen_lds_bytes(screen_plan(bs, R)) <= kScrLdsMax; }
+inline bool screen_fits(int bs, int R) { return R < 1024 && screen_lds_bytes(screen_geom(bs, R, screen_nt(bs, R))) <= kScrLdsMax; }
 
 }  // namespace vszk
