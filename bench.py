@@ -295,7 +295,7 @@ def bench_batch(args):
                       "config": {"workload": "64 Gray planes, sizes {320..3840}x{240..2160} (seed 4), sigma U[1,20], "
                                              "two-pass, bs 4, R 12, extractor 3, one hipGraph per run",
                                  "mpix": round(px / 1e6, 2), "schedule": chosen,
-                                 "matcher": matcher,
+                                 "matcher": "screen" if b.screened() else matcher,
                                  "staged_ms": sched_ms["staged"], "persistent_ms": sched_ms["persistent"],
                                  "sequential_ms": round(dt_seq * 1e3, 3),
                                  "sequential_mpix_s": round(px / dt_seq / 1e6, 3),
@@ -656,7 +656,7 @@ def main():
                    "sigma": SIGMA, "path": "plain FP32", **{k: v for k, v in PARAMS.items()},
                    "psnr_y_db": round(psnr_y, 3), "psnr_yuv_db": [round(v, 3) for v in psnr_planes],
                    "match_ms_per_step": round(t_match * 1e3, 4), "basic_pass_ms": round(t_basic * 1e3, 4),
-                   "matcher": device.match_plan(kp_b),
+                   "matcher": "screen" if device.match_screened(kp_b) else device.match_plan(kp_b),
                    "filter_tiles": {"basic": list(device.filter_plan(kp_b)), "wiener": list(device.filter_plan(kp_f))}},
         "roofline": {"bound": "mfma", "achieved": round(screen, 3), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(screen / PEAK_BF16_TFLOPS, 4), "traffic": traffic,

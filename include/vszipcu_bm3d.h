@@ -75,12 +75,10 @@ size_t vsz_bm3d_workspace_size(const vsz_bm3d_kparams *p);
 int vsz_bm3d_match(const vsz_bm3d_kparams *p, const float *d_img, int32_t *d_matches, void *stream);
 
 /* Diagnostic, no reference counterpart: the exhaustive matcher of vsz_bm3d_match for these
- * parameters: "lds4" (shared-column, block_step 4), "lds_rows1/2/4" (LDS-staged, search rows split
+ * parameters, which runs unless vsz_bm3d_match_screened (vszipcu_plan.h) says otherwise: "lds4" (shared-column, block_step 4), "lds_rows1/2/4" (LDS-staged, search rows split
  * over 1, 2 or 4 lanes), "lds_short" (LDS-staged 16 x 8-block tile) or "global" (raw buffer loads,
  * windows beyond the LDS budget); "+temporal" when radius > 0 (centre frame, then the predictive
- * search). Spatial and centre-frame ssd searches with a bm_range of 12 to 16 or more (9 or more
- * on small planes) whose windows fit its LDS budget run as a screened search on the matrix cores in
- * its place, with the same lists and distances. "" for invalid parameters. The returned string is static. */
+ * search). "" for invalid parameters. The returned string is static. */
 const char *vsz_bm3d_match_plan(const vsz_bm3d_kparams *p);
 
 /* Diagnostic, no reference counterpart: the filter vsz_bm3d_run would launch for these

@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "vszipcu_bm3d.h"
+#include "vszipcu_plan.h"
 #include "internal.h"
 #include "screen_geom.h"
 
@@ -3284,6 +3285,20 @@ bool screened(const MatchArgs &a, int metric) {
            screen_pays(a.block_step, a.bm_range, (long long)((a.nbx + 3) / 4) * ((a.nby + 3) / 4), a.block_step == 4 && (a.width - 8) % 4 == 0);
 }
 
+// What the choice of a search kernel depends on.
+MatchArgs plan_args(const vsz_bm3d_kparams *p) {
+    const Layout L = layout_of(p);
+    MatchArgs m{};
+    m.width = p->width;
+    m.height = p->height;
+    m.stride = p->stride;
+    m.nbx = L.nbx;
+    m.nby = L.nby;
+    m.block_step = p->block_step;
+    m.bm_range = p->bm_range;
+    return m;
+}
+
 struct MatchPlan {
     MatchKernel kernel;
     size_t lds;
@@ -3636,17 +3651,14 @@ const char *vsz_bm3d_match_plan(const vsz_bm3d_kparams *p) {
         vsz_fail(VSZ_EINVAL, "invalid kernel parameters");
         return "";
     }
-    const Layout L = layout_of(p);
-    MatchArgs m{};
-    m.width = p->width;
-    m.height = p->height;
-    m.stride = p->stride;
-    m.nbx = L.nbx;
-    m.nby = L.nby;
-    m.block_step = p->block_step;
-    m.bm_range = p->bm_range;
-    const MatchPlan pl = plan_match(m, p->metric);
+    const MatchPlan pl = plan_match(plan_args(p), p->metric);
     return p->radius > 0 ? temporal_names[pl.kernel] : names[pl.kernel];
+}
+
+int vsz_bm3d_match_screened(const vsz_bm3d_kparams *p, int *screen) {
+    if (!kparams_ok(p) || !screen) return vsz_fail(VSZ_EINVAL, "vsz_bm3d_match_screened: invalid arguments");
+    *screen = screened(plan_args(p), p->metric) ? 1 : 0;
+    return VSZ_OK;
 }
 
 int vsz_bm3d_filter_plan(const vsz_bm3d_kparams *p, int *tbx, int *tby, int *per_cu) {
@@ -4605,6 +4617,12 @@ int vsz_bm3d_batch_schedule(const vsz_bm3d_batch *b, int *schedule, int *shared_
     if (!b || !schedule || !shared_cols) return vsz_fail(VSZ_EINVAL, "vsz_bm3d_batch_schedule: invalid arguments");
     *schedule = b->schedule;
     *shared_cols = b->global_match ? 2 : b->shared_cols ? 1 : 0;
+    return VSZ_OK;
+}
+
+int vsz_bm3d_batch_screened(const vsz_bm3d_batch *b, int *screen) {
+    if (!b || !screen) return vsz_fail(VSZ_EINVAL, "vsz_bm3d_batch_screened: invalid arguments");
+    *screen = b->screen() ? 1 : 0;
     return VSZ_OK;
 }
 

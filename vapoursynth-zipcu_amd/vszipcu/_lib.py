@@ -138,6 +138,12 @@ PROTOTYPES = {
     "vsz_filter_free": (None, [C.c_void_p]),
 }
 
+# include/vszipcu_plan.h
+PLAN_PROTOTYPES = {
+    "vsz_bm3d_match_screened": (C.c_int, [C.POINTER(KParams), C.POINTER(C.c_int)]),
+    "vsz_bm3d_batch_screened": (C.c_int, [C.c_void_p, C.POINTER(C.c_int)]),
+}
+
 _lib = None
 
 
@@ -148,7 +154,7 @@ def load():
         if not os.path.exists(LIB_PATH):
             raise OSError(f"libvszipcu_amd.so is not built ({LIB_PATH}); run `make -C vapoursynth-zipcu_amd`")
         L = C.CDLL(LIB_PATH)
-        for name, (res, args) in PROTOTYPES.items():
+        for name, (res, args) in (*PROTOTYPES.items(), *PLAN_PROTOTYPES.items()):
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args

@@ -66,11 +66,20 @@ def num_blocks(p: _lib.KParams):
 
 
 def match_plan(p: _lib.KParams) -> str:
-    """Name of the exhaustive matcher of vsz_bm3d_match for these parameters (no GPU needed)."""
+    """Name of the exhaustive matcher of vsz_bm3d_match for these parameters, which it launches unless
+    match_screened (no GPU needed)."""
     name = _lib.load().vsz_bm3d_match_plan(C.byref(p)).decode()
     if not name:
         raise RuntimeError(f"vszipcu: {_lib.last_error()}")
     return name
+
+
+def match_screened(p: _lib.KParams) -> bool:
+    """Whether the screened search takes the spatial (or centre-frame) search in the place of match_plan's matcher (no GPU
+    needed)."""
+    n = C.c_int()
+    _check(_lib.load().vsz_bm3d_match_screened(C.byref(p), C.byref(n)))
+    return bool(n.value)
 
 
 def filter_plan(p: _lib.KParams):
@@ -203,6 +212,13 @@ class Batch:
         sch, m = C.c_int(), C.c_int()
         _check(_lib.load().vsz_bm3d_batch_schedule(self._h, C.byref(sch), C.byref(m)))
         return {0: "staged", 1: "persistent"}[sch.value], {0: "rows", 1: "shared-column", 2: "global"}[m.value]
+
+    def screened(self) -> bool:
+        """Whether the batch searches with the screened search in the place of schedule()'s matcher; final after its
+        first run."""
+        n = C.c_int()
+        _check(_lib.load().vsz_bm3d_batch_screened(self._h, C.byref(n)))
+        return bool(n.value)
 
     def tile(self, plane: int, pass_: int):
         tx, ty = C.c_int(), C.c_int()
