@@ -137,7 +137,9 @@ typedef struct vsz_bm3d_batch_params {
     int two_pass;                /* 1: basic, then Wiener with ref = basic; 0: basic only */
     int autotune;                /* 1: on the first run, time every fitting filter tile shape per
                                     plane shape, and whole runs of every allowed (schedule, matcher)
-                                    pair, and keep the fastest; 0: cost model and preferences */
+                                    pair (with ssd windows that the screened search takes: it and one
+                                    other matcher for the staged schedule), and keep the fastest;
+                                    0: cost model and preferences */
     int schedule;                /* VSZ_BATCH_STAGED: one launch per stage (zeroing, matching,
                                     filtering, finishing of all planes, per pass) in one graph;
                                     VSZ_BATCH_PERSISTENT: the whole batch in one persistent launch

@@ -27,3 +27,25 @@ def test_batch_reports_its_search(torch_gpu, schedule, bm_range, metric, screene
     b, _ = _run(torch_gpu, PLANES, bm_range=bm_range, metric=metric, schedule=schedule, autotune=False)
     assert b.schedule() == (schedule, "rows")     # the exhaustive matcher
     assert b.screened() is screened
+
+
+def test_small_planes_screen_together(orc, torch_gpu):
+    """The rule sees all planes' tiles, since they are one launch: few enough for the screened search from bm_range 9."""
+    print("batch search: small planes R=9", flush=True)
+    b, outs = _run(torch_gpu, PLANES, bm_range=9, schedule="staged", autotune=False, two_pass=False)
+    assert b.screened()
+    for i, ((w, h, _, sg), out) in enumerate(zip(PLANES, outs)):
+        op = orc.make_params(w, h, sigma=tuple(device.scaled_sigma([sg] * 3, False)), block_step=4, bm_range=9, extractor_exp=3)
+        res, _, _ = orc.bm3d(op, synth.noisy(synth.clean_luma(w, h, i), sg, i + 9)[None, None, None])
+        assert np.array_equal(out, orc.aggregate(res[:, 0], w)[0])
+
+
+@pytest.mark.parametrize("schedule", ["staged", "auto"])
+@pytest.mark.parametrize("planes", [PLANES, PLANES[1:]])      # with and without the shared-column matcher among the pairs
+def test_tuned_batches_give_the_same(torch_gpu, planes, schedule):
+    print(f"batch search: tuned {schedule}, {len(planes)} planes", flush=True)
+    _, want = _run(torch_gpu, planes, bm_range=12, schedule="staged", autotune=False)
+    b, got = _run(torch_gpu, planes, bm_range=12, schedule=schedule, autotune=True)
+    assert b.schedule()[0] == "staged" or not b.screened()
+    for a, c in zip(want, got):
+        assert np.array_equal(a, c)

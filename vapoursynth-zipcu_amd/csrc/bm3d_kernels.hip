@@ -31,6 +31,7 @@
 
 #include "vszipcu_bm3d.h"
 #include "vszipcu_plan.h"
+#include "batch_pairs.h"
 #include "internal.h"
 #include "screen_geom.h"
 
@@ -3987,7 +3988,8 @@ struct vsz_bm3d_batch {
     bool shared_cols = false;  // every plane takes the shared-column block_step-4 matcher
     bool sc_allowed = false;   // ... may take it (the autotuner then times both matchers)
     bool global_match = false;  // windows beyond the LDS matchers' budget: the global-memory matcher
-    bool screen_ok = false;     // the staged schedule searches with the screened kernel (as `screened` for one plane)
+    bool screen_ok = false;     // the staged schedule may search with the screened kernel (as `screened`, for all planes' tiles)
+    bool use_screen = false;    // ... and does
     bool direct_filter = false; // a region beyond the filter tiles' LDS budget: direct-atomic filtering
     size_t lds_rows = 0, lds_sc = 0;
     int stride_rows = 0, stride_sc = 0;
@@ -4039,7 +4041,7 @@ struct vsz_bm3d_batch {
             for (const auto &pl : planes) m = std::max(m, pl.tile[pass].lds_bytes);
         return m;
     }
-    bool screen() const { return screen_ok && schedule == VSZ_BATCH_STAGED; }
+    bool screen() const { return use_screen && schedule == VSZ_BATCH_STAGED; }
     int match_tiles_x(const BatchPlane &pl) const {
         if (screen()) return (pl.L.nbx + 3) / 4;
         return global_match ? (pl.L.nbx + 7) / 8 : shared_cols ? (pl.L.nbx + 14) / 15 : (pl.L.nbx + 15) / 16;
@@ -4178,6 +4180,11 @@ struct vsz_bm3d_batch {
         }
     }
 
+    void use_pair(const BatchPair &p) {
+        use_matcher(p.shared_cols);
+        use_screen = p.screen;
+        schedule = p.schedule;
+    }
     void use_matcher(bool sc) {
         shared_cols = sc;
         match_lds = sc ? lds_sc : lds_rows;
@@ -4348,30 +4355,13 @@ int vsz_bm3d_batch::tune(const float *const *noisy, char *work, hipStream_t s) {
     return rc;
 }
 
-// Chooses the schedule (one persistent launch or one launch per stage) and, where every plane
-// allows the shared-column matcher, the matcher: with autotune, by timing whole runs of every
-// allowed pair on this data (one warm-up, then the best of two); otherwise by preference.
+// Chooses the schedule (one persistent launch or one launch per stage) and the search: with autotune, by timing whole runs of
+// every pair of batch_pairs on this data (one warm-up, then the best of two); otherwise by preference.
 int vsz_bm3d_batch::tune_schedule(const float *const *noisy, float *const *dst, char *work, hipStream_t s) {
-    struct Cand {
-        int sched;
-        bool sc;
-    };
-    std::vector<Cand> cands;
-    if (global_match) cands.push_back({VSZ_BATCH_STAGED, false});  // the only form for such windows
-    for (int sc = 1; sc >= 0 && !global_match; --sc) {
-        if (sc ? !sc_allowed : lds_rows == 0) continue;
-        if (bp.schedule != VSZ_BATCH_STAGED && persist_ok) cands.push_back({VSZ_BATCH_PERSISTENT, sc != 0});
-        if (bp.schedule != VSZ_BATCH_PERSISTENT) cands.push_back({VSZ_BATCH_STAGED, sc != 0});
-    }
-    if (cands.empty()) return vsz_fail(VSZ_EINVAL, "vsz_bm3d_batch_run: no schedule fits these parameters");
-    if (!bp.autotune || cands.size() == 1) {
-        // preference: the shared-column matcher, the persistent launch only where asked for
-        Cand pick = cands[0];
-        for (const Cand &c : cands)
-            if (c.sc == cands[0].sc && c.sched == (bp.schedule == VSZ_BATCH_PERSISTENT ? VSZ_BATCH_PERSISTENT : VSZ_BATCH_STAGED))
-                pick = c;
-        use_matcher(pick.sc);
-        schedule = pick.sched;
+    const std::vector<BatchPair> pairs = batch_pairs(bp.schedule, lds_rows != 0, sc_allowed, global_match, screen_ok, persist_ok);
+    if (pairs.empty()) return vsz_fail(VSZ_EINVAL, "vsz_bm3d_batch_run: no schedule fits these parameters");
+    if (!bp.autotune || pairs.size() == 1) {
+        use_pair(batch_preferred(pairs, bp.schedule));
         return VSZ_OK;
     }
     hipEvent_t e0, e1;
@@ -4379,10 +4369,9 @@ int vsz_bm3d_batch::tune_schedule(const float *const *noisy, float *const *dst, 
         return vsz_fail(VSZ_EDEVICE, "vsz_bm3d_batch_run: hipEventCreate failed");
     int rc = VSZ_OK;
     float best_ms = -1.0f;
-    Cand best = cands[0];
-    for (const Cand &c : cands) {
-        use_matcher(c.sc);
-        schedule = c.sched;
+    BatchPair best = pairs[0];
+    for (const BatchPair &c : pairs) {
+        use_pair(c);
         rc = upload(noisy, dst, work, s);
         float ms = -1.0f;
         for (int rep = 0; rep < 3 && rc == VSZ_OK; ++rep) {
@@ -4403,8 +4392,7 @@ int vsz_bm3d_batch::tune_schedule(const float *const *noisy, float *const *dst, 
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    use_matcher(best.sc);
-    schedule = best.sched;
+    use_pair(best);
     return rc;
 }
 
@@ -4439,8 +4427,6 @@ int vsz_bm3d_batch_create(const vsz_bm3d_batch_params *bp, const vsz_bm3d_plane 
         b->sc_allowed = b->lds_sc != 0;
     }
     b->global_match = !b->lds_rows && !b->sc_allowed;  // windows beyond the LDS matchers' budget
-    b->screen_ok = bp->metric == 0 && !b->global_match && screen_pays(bp->block_step, bp->bm_range, LLONG_MAX, b->sc_allowed);
-    for (int i = 0; i < n; ++i) b->screen_ok = b->screen_ok && planes[i].stride < kScrStrides;
     b->use_matcher(b->sc_allowed);
     const float fac[2] = {bits_float(0x3f021bb6u), bits_float(0x3e40c0c1u)};  // src/bm3d.zig:1013-1024
     size_t acc = 0, rest = 0;
@@ -4479,6 +4465,14 @@ int vsz_bm3d_batch_create(const vsz_bm3d_batch_params *bp, const vsz_bm3d_plane 
         acc += (pl.L.acc_bytes + 255) & ~size_t(255);
         b->planes.push_back(pl);
     }
+    // all planes' tiles are one launch
+    long long tiles = 0;
+    b->screen_ok = bp->metric == 0 && !b->global_match;
+    for (const BatchPlane &pl : b->planes) {
+        tiles += (long long)((pl.L.nbx + 3) / 4) * ((pl.L.nby + 3) / 4);
+        b->screen_ok = b->screen_ok && pl.k[0].stride < kScrStrides;
+    }
+    b->screen_ok = b->screen_ok && screen_pays(bp->block_step, bp->bm_range, tiles, b->sc_allowed);
     // the persistent form: exact aggregation, ssd or sad, dct, the LDS matchers and filter tiles
     b->persist_ok = b->exact && (bp->metric == 0 || bp->metric == 1) && bp->t2d == 0 && !b->global_match &&
                     !b->direct_filter;
