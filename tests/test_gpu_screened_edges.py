@@ -48,3 +48,19 @@ def test_wide_stride(orc, torch_gpu, stride):
     plane[0, :, :W] = torch.from_numpy(img).cuda()
     om, oe = orc.match(op, img[None])
     assert_matches_equal(_match(torch, kp, plane), om, oe)
+
+
+@pytest.mark.parametrize("bs,rng", [(4, 16), (8, 20)])
+@pytest.mark.parametrize("level", [1.0, 50.0])
+def test_isolated_bright_pixels(orc, torch_gpu, bs, rng, level):
+    """Pixels far above a window of low contrast: one term of a product outweighs the others, and the window's halves have
+    coarse steps."""
+    torch = torch_gpu
+    print(f"screened search: bright pixels {level} bs={bs} R={rng}", flush=True)
+    W, H = 132, 110
+    r = np.random.default_rng(4)
+    img = (0.2 + r.normal(0, 0.002, (H, W))).astype(np.float32)
+    img[r.integers(0, H, 12), r.integers(0, W, 12)] = level
+    kp, op = kp_and_op(orc, W, H, bs=bs, rng=rng)
+    om, oe = orc.match(op, img[None])
+    assert_matches_equal(_match(torch, kp, torch.from_numpy(img[None]).cuda()), om, oe)

@@ -862,8 +862,8 @@ __global__ __launch_bounds__(256) void k_match_lds4(MatchArgs a) {
 // ---- screened search (ssd) ---------------------------------------------------------------------
 // The distance of a block to a candidate is |a|^2 + |b|^2 - 2 a.b, and a.b over all candidates of a
 // block is a matrix product. The screen computes it on the matrix cores from half-precision copies
-// of the pixels, derives per block a threshold that every one of its 8 best candidates is proven to
-// pass (about 9 of 1089 do on video with noise), and only those are evaluated exactly, in FP32 and in
+// of the pixels, derives per block a threshold that every one of its 8 best candidates passes under the bounds
+// below (about 9 of 1089 do on video with noise), and only those are evaluated exactly, in FP32 and in
 // the reference's order of operations. Lists and distances are those of the exhaustive scan.
 //
 // A workgroup is one wave and owns 4 x 4 blocks (the 16 rows of a product). Products run on
@@ -879,10 +879,11 @@ __global__ __launch_bounds__(256) void k_match_lds4(MatchArgs a) {
 // rounded to half (subnormal halves may count as 0), with d = half a step of the largest half that the
 // block or a candidate this near can hold (screen_eps). With S the distance of two patches and S_q that of their rounded copies,
 // |sqrt(S) - sqrt(S_q)| <= 2 sqrt(64) d = eps. A computed S' = n_a - 2 (a.b - n_b/2) differs from S_q
-// by the accumulation's rounding. One product instruction was measured to be off by at most 9.3 units
-// of 2^-24 of its largest term or result (one term 2^12 times the other 31, all truncated; 2 to 4 for terms of
-// like size); 17 is what truncating every term at half a unit gives, and 3 instructions make
-// |S' - S_q| <= c (n_a + n_b) with c = 8e-6, the norms' own rounding included, and n_b <= 2 n_a + 2 S_q.
+// by the accumulation's rounding, which the instruction set does not specify: c is measured, with a margin. One product
+// instruction was off by at most 9.3 units of 2^-24 of its largest term or result (one term 2^12 times the other 31, all
+// truncated; 2 to 4 for terms of like size); 17 is what truncating every term at half a unit gives, and 3 instructions make
+// |S' - S_q| <= c (n_a + n_b) with c = 8e-6, the norms' own rounding included, and n_b <= 2 n_a + 2 S_q. The
+// chained products are held to it by a test (tests/test_gpu_mfma_error.py: 3.7e-7 (n_a + n_b) at most).
 // Pass 1 finds a T' that 8 distinct candidates do not exceed; their exact distances, hence the 8
 // best, are below (sqrt((T' + 3c n_a)(1 + 3c)) + eps)^2, up to FP32 rounding; a candidate below that has
 // S' <= T'' (screen_limit). Pass 2 recomputes the products and passes on candidates with S' <= T''.
