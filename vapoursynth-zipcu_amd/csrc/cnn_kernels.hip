@@ -95,6 +95,11 @@ __global__ __launch_bounds__(256) void k_conv3x3(const unsigned short *__restric
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane & 15, g = lane >> 4;
     const int r0 = wave * 4, o = g * 8;
+    uint4 v[kHaloPer];
+    int tile = blockIdx.x;
+    if (tile < tiles) halo_load(x, tile / (tx_n * ty_n), H, W, (tile % tx_n) * TILE, ((tile / tx_n) % ty_n) * TILE, v);
+    // after the first halo's loads, so that they arrive while it is stored: where a workgroup has one tile they were waited for
+    // (one 480x270 image, a layer: 8.5 us before the halo's, 7.9 after, 8.0 with 16 channels a wave, half the weights)
     bf16x8 wa[2][9];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -106,9 +111,6 @@ __global__ __launch_bounds__(256) void k_conv3x3(const unsigned short *__restric
 #pragma unroll
         for (int q = 0; q < 8; ++q) bo[q] = bias[mode == 1 ? 0 : o + q];
 
-    uint4 v[kHaloPer];
-    int tile = blockIdx.x;
-    if (tile < tiles) halo_load(x, tile / (tx_n * ty_n), H, W, (tile % tx_n) * TILE, ((tile / tx_n) % ty_n) * TILE, v);
     for (; tile < tiles; tile += gridDim.x) {
         const int n = tile / (tx_n * ty_n), x0 = (tile % tx_n) * TILE, y0 = ((tile / tx_n) % ty_n) * TILE;
         __syncthreads();  // every wave is done with the previous tile's halo
