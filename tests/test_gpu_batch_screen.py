@@ -49,3 +49,13 @@ def test_tuned_batches_give_the_same(torch_gpu, planes, schedule):
     assert b.schedule()[0] == "staged" or not b.screened()
     for a, c in zip(want, got):
         assert np.array_equal(a, c)
+
+
+def test_large_shared_column_planes_screen_only_if_timed(torch_gpu):
+    """Above 2048 tiles the shared-column scan is preferred at bm_range 12; the autotuner may find the screen faster."""
+    print("batch search: shared columns, 960x720", flush=True)
+    planes = [(960, 720, 960, 8.0)]
+    b, want = _run(torch_gpu, planes, bm_range=12, schedule="staged", autotune=False)
+    assert b.schedule() == ("staged", "shared-column") and not b.screened()
+    b, got = _run(torch_gpu, planes, bm_range=12, schedule="staged", autotune=True)
+    assert np.array_equal(want[0], got[0])

@@ -3269,6 +3269,7 @@ int tied_wgs(int tiles) { return (int)std::min(4LL * tiles, 1024LL); }
 //   up to 512   8/12 at 960x540: 0.66 and 1.10; 6/12 at 640x360: 0.50 and 0.86 (not 8/9: 0.80 and 1.40, 6/9: 0.80 and 1.33)
 //   above       4/12 at 640x360: 0.50 and 0.93; 6/12 at 1920x1080: 0.54 and 0.90; 2/12: 0.41 and 0.57; 4/16: 0.49 and 0.71, at
 //               3840x2160 0.55 and 1.28 (not 4/9 at 640x360: 0.65 and 1.33, 3/9: 0.76 and 1.51)
+//   (6/12 at 1280x720: 0.58 and 1.28)
 //   the shared-column scan is twice as fast above 2048 tiles   (not 4/12 at 1280x720: 0.78 and 1.26, 2560x1440: 0.80 and 1.38,
 //               3840x2160: 0.83 and 1.76)
 //   beyond an eighth of a CU's LDS   8/16 at 1280x720 (920 tiles): 0.55 and 1.11; 6/16 at 1920x1080: 0.55 and 0.84; 4/20: 0.58 and
@@ -3280,6 +3281,12 @@ bool screen_pays(int bs, int R, long long tiles, bool shared) {
     const ScreenGeom G = screen_plan(bs, R, tiles);
     if (screen_lds_bytes(G) > kScrLds8) return R >= 16 && (tiles <= 1024 || screen_share(G, R) >= 0.29f);
     return R >= (shared && tiles > 2048 ? 16 : 12);
+}
+
+// Whether it may gain by content: what a batch's autotuner times on its planes beside the scan. 64 planes of 320x240 to 3840x2160 at
+// block_step 4, bm_range 12, noise, all for the shared-column scan: 38.1 ms, screened 33.4.
+bool screen_may(int bs, int R) {
+    return screen_fits(bs, R) && R >= (screen_lds_bytes(screen_plan(bs, R, 1)) <= kScrLds8 ? 12 : 16);
 }
 
 bool screened(const MatchArgs &a, int metric) {
@@ -3989,7 +3996,7 @@ struct vsz_bm3d_batch {
     bool shared_cols = false;  // every plane takes the shared-column block_step-4 matcher
     bool sc_allowed = false;   // ... may take it (the autotuner then times both matchers)
     bool global_match = false;  // windows beyond the LDS matchers' budget: the global-memory matcher
-    bool screen_ok = false;     // the staged schedule may search with the screened kernel (as `screened`, for all planes' tiles)
+    bool screen_ok = false;     // the staged schedule may search with the screened kernel (by its rule for all planes' tiles, or timed)
     bool use_screen = false;    // ... and does
     bool direct_filter = false; // a region beyond the filter tiles' LDS budget: direct-atomic filtering
     size_t lds_rows = 0, lds_sc = 0;
@@ -4473,7 +4480,8 @@ int vsz_bm3d_batch_create(const vsz_bm3d_batch_params *bp, const vsz_bm3d_plane 
         tiles += (long long)((pl.L.nbx + 3) / 4) * ((pl.L.nby + 3) / 4);
         b->screen_ok = b->screen_ok && pl.k[0].stride < kScrStrides;
     }
-    b->screen_ok = b->screen_ok && screen_pays(bp->block_step, bp->bm_range, tiles, b->sc_allowed);
+    b->screen_ok = b->screen_ok && (screen_pays(bp->block_step, bp->bm_range, tiles, b->sc_allowed) ||
+                                    (bp->autotune && screen_may(bp->block_step, bp->bm_range)));
     // the persistent form: exact aggregation, ssd or sad, dct, the LDS matchers and filter tiles
     b->persist_ok = b->exact && (bp->metric == 0 || bp->metric == 1) && bp->t2d == 0 && !b->global_match &&
                     !b->direct_filter;
