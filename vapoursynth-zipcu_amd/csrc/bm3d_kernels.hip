@@ -1142,6 +1142,10 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
         bad = !(top < 1.0e37f);
         sc = bad ? 1.0f : __builtin_ldexpf(1.0f, min(10 - __builtin_amdgcn_frexp_expf(top), 120));
     }
+    // uniform values do without vector registers; what is not read in the products' loops is kept in LDS (ScreenWave) or read again.
+    // 14 registers were spilled otherwise: 1920x1080, block_step 4, bm_range 16 took 170 us, 167 without
+    big = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(big)));
+    sc = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(sc)));
     const bool flat = big == 0.0f && !bad;
     if (lane < 16) {
         ws->refpos[lane] = pack_xy(xr_n, yr_n);
@@ -1236,7 +1240,8 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
         // A: row n is the block (n & 3, n >> 2)
         scr_h8 A[4][3];
         const auto loadA = [&]() {
-            const int xr = xr_n - rx0, yr = yr_n - ry0;
+            const unsigned rp = ws->refpos[n];
+            const int xr = pos_x(rp) - rx0, yr = pos_y(rp) - ry0;
             const scr_h8 z = {};
 #pragma unroll
             for (int s = 0; s < 4; ++s)
@@ -1521,7 +1526,7 @@ __device__ __forceinline__ void match_screen_body(const MatchArgs &a, const Scre
             // leaves out those of blocks that are left and those that come after their block's 8 zero distances
             const auto drop = [&]() {
                 unsigned k0 = 0u, k1 = 0u;
-#pragma unroll
+#pragma unroll 1
                 for (int q = 0; q < 4; ++q) {
                     const unsigned b = (from >> 4) * 4u + q;
                     const unsigned long long k = ws->best[b * 8u + 7u];
