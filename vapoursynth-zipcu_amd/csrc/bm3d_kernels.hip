@@ -894,9 +894,9 @@ __global__ __launch_bounds__(256) void k_match_lds4(MatchArgs a) {
 // them nothing later can enter; a block with more candidates than ScreenGeom::block that has not ended is left to
 // k_match_tied, and so are all blocks of a tile with values that are not finite. The marks are in the match list: the third
 // component of a block row's first entry, which no list uses, holds a bit per block. 1920x1080, block_step 4, bm_range 16, scan /
-// screened in us (before: a tile with more than 384 was left as a whole, before any was evaluated): flat drawn art 335 / 166 (711),
-// ordered dither 340 / 239 (1461), text 380 / 270 (496), art with noise of sigma 1 385 / 290 (419), noise with letterbox
-// bars 358 / 198 (285), noise 355 / 174 (172).
+// screened in us (before: a tile with more than 384 was left as a whole, before any was evaluated): flat drawn art 331 / 172 (711),
+// ordered dither 338 / 227 (1461), text 378 / 256 (496), art with noise of sigma 1 384 / 272 (419), noise with letterbox
+// bars 359 / 192 (285), noise 356 / 170 (172).
 //
 // What bounds it: VALU issue, about 30 instructions per candidate row of 16 blocks in pass 1 and 40 in
 // pass 2 with the products (11 per 4 rows and 16 columns, 16 cycles each) beside them, then the latency of
